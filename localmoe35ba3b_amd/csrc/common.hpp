@@ -109,6 +109,22 @@ __device__ __forceinline__ void dequant16(u32x4 w, float s, uint32_t out[8]) {
   }
 }
 
+// Eight int8 weights -> eight T(q * s): the signed byte converts exactly
+// (v_cvt_f32_i32 with a sign-extended byte operand), so q * s is the
+// correctly rounded fp32 product, then RNE to T - bit-identical to
+// dequant8 with one operation fewer per four weights.
+template <typename T>
+__device__ __forceinline__ u32x4 dequant8s(uint2 w, float s) {
+  float f[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f[i] = (float)(int8_t)(w.x >> (8 * i)) * s;
+    f[4 + i] = (float)(int8_t)(w.y >> (8 * i)) * s;
+  }
+  return u32x4{T::pack2(f[0], f[1]), T::pack2(f[2], f[3]), T::pack2(f[4], f[5]),
+               T::pack2(f[6], f[7])};
+}
+
 // ------------------------------------------------------------ lane reductions
 // Sums over the 8 lanes of each lane octet (lanes 8j..8j+7); every lane of the
 // octet receives the total.  DPP: xor-1 and xor-2 quad permutations, then the

@@ -11,14 +11,16 @@
 // MFMA (the reference rounds the dequantized weight to the activation dtype
 // before the MMA, int8.py:21), so the MFMA consumes bit-identical operands
 // to the reference's tl.dot; only the fp32 summation order differs.
-//   w8a16_mfma_kernel    dense and generic (fp16 rows, other K): 256 threads,
+//   w8a16_mfma_kernel    dense, K other than 512, 2048 and 4096: 256 threads,
 //                        BM x 128 tile, K in 64-wide stages, weights
 //                        dequantized into LDS.
 //   grouped_mfma_kernel  routed, any K, up to 128-row tiles (large_tile).
-//   grouped_rb_kernel    routed, and dense bf16, at the model's K (2048
-//                        gate_up, 512 down) in tiles of up to 96 rows:
-//                        weights streamed straight into registers and
-//                        dequantized there.
+//   grouped_rb_kernel    routed at the model's K (2048 gate_up, 512 down) in
+//                        tiles of up to 96 rows, and dense at K = 512, 2048
+//                        and 4096 where many rows fill its tiles: weights
+//                        streamed straight into registers and dequantized
+//                        there.
+// Dense calls of fewer rows run the K-split tiles of ksplit.hip.
 // In SwiGLU mode a tile's columns pair every gate column with its up partner
 // in the same lane.
 #include <type_traits>
@@ -56,16 +58,23 @@ struct GemmArgs {
   int tile_rows;  // rows covered by one table tile (<= BM)
   int nt_count;   // column tiles
   int mt_count;   // row tiles (table rows, or dense M tiles)
+  bool cols_by_xcd;  // dense: a column tile's row tiles share an XCD, not a row tile's columns
 };
 
 // Workgroups are dealt to the 8 XCDs round-robin by linear id.  Map linear
 // id b -> (row tile, column tile) so that all column tiles of one row tile
 // run on the same XCD back to back: the gathered activation rows of a tile
 // are then read from HBM/MALL once and served from that XCD's L2 for the
-// other column tiles.  Returns false for padding workgroups.
+// other column tiles.  With cols_by_xcd (dense) the roles are swapped.
+// Returns false for padding workgroups.
 __device__ __forceinline__ bool xcd_tile(const GemmArgs &a, int &mt, int &nt) {
   const int b = blockIdx.x;
   const int j = b >> 3;
+  if (a.cols_by_xcd) {
+    mt = j % a.mt_count;
+    nt = (j / a.mt_count) * 8 + (b & 7);
+    return nt < a.nt_count;
+  }
   mt = (j / a.nt_count) * 8 + (b & 7);
   nt = j % a.nt_count;
   return mt < a.mt_count;
@@ -73,7 +82,8 @@ __device__ __forceinline__ bool xcd_tile(const GemmArgs &a, int &mt, int &nt) {
 
 // Workgroups of an XCD-mapped launch; callers reject counts beyond one
 // launch's grid (2^31 - 1) before launching.
-static int64_t xcd_grid(int64_t mtiles, int64_t ntiles) {
+static int64_t xcd_grid(int64_t mtiles, int64_t ntiles, bool cols_by_xcd = false) {
+  if (cols_by_xcd) return 8 * mtiles * ((ntiles + 7) / 8);
   return 8 * ntiles * ((mtiles + 7) / 8);
 }
 
@@ -256,22 +266,6 @@ __global__ __launch_bounds__(256) void w8a16_mfma_kernel(GemmArgs a) {
 // are prefetched into registers while the current stage computes.
 constexpr int kGBM = 128;
 constexpr int kLDB = kBK + 8;  // int8 bytes per LDS row of the weight tile
-
-// Eight int8 weights -> eight T(q * s): the signed byte converts exactly
-// (v_cvt_f32_i32 with a sign-extended byte operand), so q * s is the
-// correctly rounded fp32 product, then RNE to T - bit-identical to
-// dequant8 with one operation fewer per four weights.
-template <typename T>
-__device__ __forceinline__ u32x4 dequant8s(uint2 w, float s) {
-  float f[8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[i] = (float)(int8_t)(w.x >> (8 * i)) * s;
-    f[4 + i] = (float)(int8_t)(w.y >> (8 * i)) * s;
-  }
-  return u32x4{T::pack2(f[0], f[1]), T::pack2(f[2], f[3]), T::pack2(f[4], f[5]),
-               T::pack2(f[6], f[7])};
-}
 
 // Eight weights of the LM_TILES_F16 format (bytes u = q + 128, each dword
 // holding k = 0, 2, 1, 3 in byte order) -> eight fp16 values q, exactly, in k
@@ -983,7 +977,7 @@ static int launch_rb(GemmArgs a, unsigned mtiles, hipStream_t st) {
   constexpr int RBN = NW * TN;
   a.nt_count = SWIGLU ? (int)cdiv(a.N / 2, RBN / 2) : (int)cdiv(a.N, RBN);
   a.mt_count = (int)mtiles;
-  const int64_t grid = xcd_grid(a.mt_count, a.nt_count);
+  const int64_t grid = xcd_grid(a.mt_count, a.nt_count, a.cols_by_xcd);
   LM_REQUIRE(grid < (int64_t(1) << 31), LM_EINVAL, "problem too large for one launch");
   grouped_rb_kernel<T, SWIGLU, GATHER, WL, K, BM, TN, kRbBD, kRbHL, AD, NW, OCC>
       <<<(unsigned)grid, NW * 64, 0, st>>>(a);
@@ -996,13 +990,17 @@ template <typename T, bool SWIGLU, bool GATHER, int WL>
 static int launch_grouped(GemmArgs a, unsigned mtiles, hipStream_t st) {
   if (mtiles == 0) return LM_OK;
   if constexpr (WL == kWlDirect && !SWIGLU && !GATHER) {
-    if (!a.table && a.tile_rows == kRbBMTall && (a.K == 2048 || a.K == 512)) {
-      if ((int64_t)mtiles * cdiv(a.N, kRbNWWide * kRbTN) >= kRbWideTiles)
-        return a.K == 2048
-                   ? launch_rb<T, false, false, WL, 2048, kRbBMTall, kRbNWWide>(a, mtiles, st)
-                   : launch_rb<T, false, false, WL, 512, kRbBMTall, kRbNWWide>(a, mtiles, st);
-      return a.K == 2048 ? launch_rb<T, false, false, WL, 2048, kRbBMTall>(a, mtiles, st)
-                         : launch_rb<T, false, false, WL, 512, kRbBMTall>(a, mtiles, st);
+    if (!a.table) {  // dense rows, K = 512, 2048 or 4096
+      const bool wide = (int64_t)mtiles * cdiv(a.N, kRbNWWide * kRbTN) >= kRbWideTiles;
+      auto go = [&](auto k_tag) -> int {
+        constexpr int KC = decltype(k_tag)::value;
+        if (a.tile_rows != kRbBMTall) return launch_rb<T, false, false, WL, KC>(a, mtiles, st);
+        return wide ? launch_rb<T, false, false, WL, KC, kRbBMTall, kRbNWWide>(a, mtiles, st)
+                    : launch_rb<T, false, false, WL, KC, kRbBMTall>(a, mtiles, st);
+      };
+      if (a.K == 4096) return go(std::integral_constant<int, 4096>{});
+      if (a.K == 2048) return go(std::integral_constant<int, 2048>{});
+      return go(std::integral_constant<int, 512>{});
     }
   }
   if (a.tile_rows <= 96 && (a.K == 2048 || a.K == 512))
@@ -1042,13 +1040,30 @@ int w8a16_gemm_dense(const void *x, const int8_t *q, const float *s, void *y, in
   a.N = (int)n;
   a.K = (int)k;
   (void)large_tile;
-  // Rows at the model's K: the register-streamed kernel over 96-row tiles of
-  // the dense matrix (128-row tiles from kDenseTallM rows; no tile table),
-  // faster than the LDS-dequant kernel because each wave dequantizes only
-  // its own columns' weights.
-  if (k == 2048 || k == 512) {
+  // K = 512, 2048 or 4096: small tiles whose waves split K (ksplit.hip) or the
+  // register-streamed kernel over 96-row tiles (128-row tiles from
+  // kDenseTallM rows; no tile table), whichever is estimated to be faster.  A
+  // 96 x 128 tile walks K alone and takes about 21.5 us at K = 2048 (8.5 us
+  // with its launch at 512, 41 us at 4096) whether one or 256 of them run;
+  // each further round of 256 tiles adds about half of that.  The K-split tiles take 4 to
+  // 20 us while one or two rounds of them hold the matrix (x [45, 2048] by
+  // [4096, 2048]: 6.9 against 20.5 us; [333, 4096] by [2048, 4096]: 17
+  // against 41), and lose where the rows fill the tall tiles ([700, 2048] by
+  // [4096, 2048]: 30 against 24 us).  Other K keeps the LDS-dequant kernel.
+  const KsPlan plan = ksplit_plan(m, n, k);
+  if (plan.shape >= 0) {
     const int bm = m >= kDenseTallM ? kRbBMTall : 96;
+    const int64_t rounds = ((int64_t)cdiv(m, bm) * cdiv(n, kRbNW * kRbTN) + 255) / 256;
+    const double rb_cost = (2.0 + 19.5 * (double)k / 2048.0) * (0.55 + 0.45 * (double)rounds);
+    if (plan.cost <= rb_cost) return w8a16_ksplit(plan, x, q, s, y, m, n, k, dtype, st);
     a.tile_rows = bm;
+    // All row tiles of a column tile on one XCD: every XCD has work whatever
+    // the number of row tiles, and reads only its part of the weights
+    // ([100, 2048] by [8192, 2048]: 22.8 us against 31.3 with a row tile's
+    // columns on one XCD; [2048, 2048] by [8192, 2048]: 76 against 82).  Whole
+    // rounds of row tiles with at least as many bytes as the weights keep
+    // their columns together ([2048, 2048] by [4096, 2048]: 38.9 against 39.2).
+    a.cols_by_xcd = n > 2 * m || cdiv(m, bm) % 8 != 0;
     return dtype == LM_BF16 ? launch_grouped<BF16, false, false, kWlDirect>(a, cdiv(m, bm), st)
                             : launch_grouped<FP16, false, false, kWlDirect>(a, cdiv(m, bm), st);
   }
@@ -1130,7 +1145,17 @@ extern "C" int lm_w8a16_linear(const void *x, const int8_t *q, const float *s, v
              "Invalid INT8 group geometry");
   if (m == 0) return LM_OK;
   LM_REQUIRE(x && q && s && y, LM_EINVAL, "null pointer");
-  if (m <= 8) return w8a16_gemv_dense(x, q, s, y, m, n, k, dtype, as_stream(stream));
+  if (m <= 8) {
+    // One or two rows stream the weights through the GEMV (lm_head
+    // [248320, 2048]: 77 against 92 us on K-split tiles); from three rows on
+    // the GEMV's dot products cost more than the weights (200 against 93 us;
+    // at N = 4096 and 8 rows 6.9 against 4.1 us), and at K = 512 one round of
+    // K-split tiles is the shorter chain (2.6 against 3.4 us).
+    const KsPlan plan = ksplit_plan(m, n, k);
+    if (plan.shape >= 0 && (m > 2 || (k == 512 && n <= 256 * 16)))
+      return w8a16_ksplit(plan, x, q, s, y, m, n, k, dtype, as_stream(stream));
+    return w8a16_gemv_dense(x, q, s, y, m, n, k, dtype, as_stream(stream));
+  }
   LM_REQUIRE(m < (1LL << 31), LM_EINVAL, "Invalid INT8 group geometry");
   return w8a16_gemm_dense(x, q, s, y, m, n, k, dtype, large_tile, as_stream(stream));
 }

@@ -381,17 +381,22 @@ static int launch_w8a16(const GemvArgs &a, unsigned gy, hipStream_t st) {
   const size_t lds = (size_t)MT * a.K * 2 + (size_t)a.RB * G * 4 + (size_t)MT * a.RB * G * 4;
   LM_REQUIRE(lds <= 160 * 1024, LM_EINVAL, "Invalid INT8 group geometry");
   const dim3 grid(cdiv(a.N, a.RB), gy);
-  const bool large = gemv_large_blocks((int64_t)grid.x * gy, MT);
-  if (a.K == 2048 && large)
-    w8a16_gemv_kernel<T, MT, 2048, kGemvThreadsK><<<grid, kGemvThreadsK, lds, st>>>(a);
-  else if (a.K == 2048)
-    w8a16_gemv_kernel<T, MT, 2048, kGemvThreads><<<grid, kGemvThreads, lds, st>>>(a);
-  else if (a.K == 512 && large)
-    w8a16_gemv_kernel<T, MT, 512, kGemvThreadsK><<<grid, kGemvThreadsK, lds, st>>>(a);
-  else if (a.K == 512)
-    w8a16_gemv_kernel<T, MT, 512, kGemvThreads><<<grid, kGemvThreads, lds, st>>>(a);
-  else
+  // three or more rows at these K run the K-split tiles (lm_w8a16_linear)
+  if constexpr (MT <= 2) {
+    const bool large = gemv_large_blocks((int64_t)grid.x * gy, MT);
+    if (a.K == 2048 && large)
+      w8a16_gemv_kernel<T, MT, 2048, kGemvThreadsK><<<grid, kGemvThreadsK, lds, st>>>(a);
+    else if (a.K == 2048)
+      w8a16_gemv_kernel<T, MT, 2048, kGemvThreads><<<grid, kGemvThreads, lds, st>>>(a);
+    else if (a.K == 512 && large)
+      w8a16_gemv_kernel<T, MT, 512, kGemvThreadsK><<<grid, kGemvThreadsK, lds, st>>>(a);
+    else if (a.K == 512)
+      w8a16_gemv_kernel<T, MT, 512, kGemvThreads><<<grid, kGemvThreads, lds, st>>>(a);
+    else
+      w8a16_gemv_kernel<T, MT, 0, kGemvThreads><<<grid, kGemvThreads, lds, st>>>(a);
+  } else {
     w8a16_gemv_kernel<T, MT, 0, kGemvThreads><<<grid, kGemvThreads, lds, st>>>(a);
+  }
   return check_launch("w8a16_gemv_kernel");
 }
 

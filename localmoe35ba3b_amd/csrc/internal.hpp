@@ -41,4 +41,15 @@ struct RoutedGemm {
 };
 int routed_gemm(const RoutedGemm &r, hipStream_t st);
 
+// Dense W8A16 over small tiles whose waves split K (ksplit.hip): the tile
+// shape for an [m, n, k] problem (shape < 0: k not served) with its estimated
+// time in us, and the launch.
+struct KsPlan {
+  int shape;
+  double cost;
+};
+KsPlan ksplit_plan(int64_t m, int64_t n, int64_t k);
+int w8a16_ksplit(const KsPlan &plan, const void *x, const int8_t *q, const float *s, void *y,
+                 int64_t m, int64_t n, int64_t k, int dtype, hipStream_t st);
+
 }  // namespace lm

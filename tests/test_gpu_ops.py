@@ -186,6 +186,30 @@ def test_w8a16_linear_exact(dev, m, n):
     assert np.array_equal(npf(y), O.bf16(exact.astype(np.float32)))
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('m,n,k', [
+    (1, 40, 512), (3, 1000, 512), (33, 4090, 512), (97, 4080, 512), (700, 2048, 512),
+    (3, 16, 2048), (5, 4104, 2048), (8, 9000, 2048), (16, 17, 2048), (100, 1000, 2048),
+    (129, 4096, 2048), (700, 1030, 2048), (700, 4100, 2048),
+    (3, 1000, 4096), (17, 600, 4096), (65, 2050, 4096), (260, 2040, 4096), (1100, 300, 4096),
+    (1057, 4096, 4096), (2000, 4100, 4096)])
+def test_w8a16_linear_ksplit_exact(dev, m, n, k, dtype):
+    """Every K-split tile shape at each K it serves (16 to 96 rows by 16 to 64
+    columns, ragged in both), and the tall tiles at K = 4096: integers and
+    powers of two make every sum exact in fp32 (below 2^24 units of 2^-6), so
+    the result is the rounded exact product whatever the order of the sum."""
+    g = np.random.default_rng(m + n + k)
+    x = g.integers(-8, 9, size=(m, k)).astype(np.float32)
+    q = g.integers(-127, 128, size=(n, k)).astype(np.int8)
+    s = np.full((n, k // 128), 2.0 ** -6, np.float32)
+    s[::3, ::2] = 2.0 ** -5
+    y = int8.linear(torch.from_numpy(x).to(dtype).to(dev), torch.from_numpy(q).to(dev),
+                    torch.from_numpy(s).to(dev))
+    w = q.astype(np.float32).reshape(n, -1, 128) * s[..., None]
+    exact = torch.from_numpy(x) @ torch.from_numpy(w.reshape(n, k)).t()
+    assert torch.equal(y.cpu(), exact.to(dtype))
+
+
 @pytest.mark.parametrize('m', [64, 1030])
 def test_w8a16_linear_fp16(dev, m):
     gen = seeded(5)
