@@ -8,11 +8,9 @@ int router_logits(const uint16_t *x, const uint16_t *w, const float *bias, float
                   int64_t T, int64_t E, int64_t H, hipStream_t st);
 int router_topk(const float *logits, int64_t T, int64_t E, int64_t K, int64_t *ids,
                 uint16_t *weights, hipStream_t st);
-// shared_rows > 0 appends cdiv(shared_rows, bm) tiles (E, R + j*bm, R + shared_rows)
-// after the max_tiles plan rows and pos[R + t] = t for the always-on shared expert.
 int route_plan(const int64_t *ids, int64_t T, int64_t K, int64_t E, int64_t bm, int64_t *pos,
                int64_t *table, int64_t max_tiles, int64_t *ordered, int64_t *slots,
-               int64_t shared_rows, hipStream_t st);
+               hipStream_t st);
 // One routed grouped W8A16 GEMM (gate_up with gather + optional SwiGLU
 // epilogue, or down over contiguous rows) over a (expert, start, stop) tile
 // table.  Table experts are clamped into [0, experts), starts and stops into

@@ -4,7 +4,7 @@
 //   device route plan: stable token sort / permute  (gpu_routes.py:17-63)
 //   ordered combines for decode and prefill         (int8.py:240-250, prefill.py:37-49)
 //   SwiGLU glue, RMSNorm                            (HF:715, HF:801-815)
-#include <type_traits>
+#include <algorithm>
 
 #include "internal.hpp"
 
@@ -179,20 +179,29 @@ int router_topk(const float *logits, int64_t T, int64_t E, int64_t K, int64_t *i
 }
 
 // ============================================================ route plan
-// Stable counting sort of the flat route ids by expert, one 1024-thread block.
-// Wave w owns a contiguous slice of the routes and walks it 64 at a time:
-// lanes holding the same expert id find each other with eight ballots over
-// the id bits, so a route's rank among equal ids inside the slice is the
-// wave's running count for that expert plus the equal ids in lower lanes.
-// A column scan over the 16 per-wave counts and a scan over experts turn
-// these slice ranks into positions of the stable order - three block
-// barriers in total.  ids are clamped into [0, E), so a malformed id can
-// never index out of bounds.
+// Stable counting sort of the flat route ids by expert, in one launch without
+// communication between workgroups.  Workgroup b ranks the routes of its own
+// tokens; to place them it needs the count of every expert over all routes
+// and over the routes before its own, which it takes itself: every workgroup
+// reads all ids (128 KB for 2048 tokens x 8, served by L2) into LDS
+// histograms.  A single workgroup had to rank all routes one 64-lane chunk
+// after the other: 40 us for 2048 x 8 and 1644 us for 60000 x 8, against 8 and
+// 102 us.  With up to 1024 routes per workgroup a wave ranks one chunk; a
+// call then costs its launch, the ids' latency and four barriers (5.0 us for
+// one slice).
+//
+// Within the slice, wave w owns a contiguous run of routes and walks it 64 at
+// a time: lanes holding the same expert id find each other with eight ballots
+// over the id bits, so a route's position is the wave's running position of
+// that expert plus the equal ids in lower lanes.  The running positions start
+// at the expert's offset, plus its routes before the slice, plus those of the
+// slice's earlier waves.  A slice holds whole tokens, and a route's place in
+// its token's ascending order is counted from the token's ids.  ids are
+// clamped into [0, E), so a malformed id can never index out of bounds.  One
+// further workgroup, without routes, writes the tile table.
 constexpr int kPlanThreads = 1024;
 constexpr int kPlanWaves = kPlanThreads / 64;
-// Routes per call whose ids and ranks are staged in LDS (ids as bytes,
-// ranks as 16-bit); larger calls keep the ranks in the `ordered` output.
-constexpr int kPlanLdsRoutes = 40960;
+constexpr int kPlanBlocks = 255;  // at most this many slices, of at least kPlanThreads routes
 
 // Exclusive scan of one value per thread over the first 256 threads of a
 // 1024-thread block (the others pass 0); returns the prefix, *total = sum.
@@ -215,75 +224,61 @@ __device__ int block_scan_256(int v, int *scratch, int *total) {
   return base + incl - v;
 }
 
-// Stable sort of up to N (id, slot, value) triples by id with an odd-even
-// transposition network (static register indices only).
-template <int N>
-__device__ __forceinline__ void sort_triples(int (&id)[N], int (&sl)[N], int (&v)[N]) {
-#pragma unroll
-  for (int pass = 0; pass < N; ++pass) {
-#pragma unroll
-    for (int i = pass & 1; i + 1 < N; i += 2) {
-      if (id[i] > id[i + 1]) {
-        const int a = id[i], b = sl[i], c = v[i];
-        id[i] = id[i + 1];
-        sl[i] = sl[i + 1];
-        v[i] = v[i + 1];
-        id[i + 1] = a;
-        sl[i + 1] = b;
-        v[i + 1] = c;
-      }
-    }
-  }
-}
-
-template <bool LDS>
 __global__ __launch_bounds__(1024) void route_plan_kernel(const int64_t *__restrict__ ids, int T,
-                                                          int K, int E, int bm,
+                                                          int K, int E, int bm, int tokens_per_block,
                                                           int64_t *__restrict__ pos,
                                                           int64_t *__restrict__ table,
                                                           int max_tiles,
                                                           int64_t *__restrict__ ordered,
-                                                          int64_t *__restrict__ slots,
-                                                          int shared_rows) {
+                                                          int64_t *__restrict__ slots) {
+  __shared__ int count[2][256];  // routes before the slice / from its start on
+  __shared__ int wpos[kPlanWaves][256];
   __shared__ int offs[257], tends[256], scratch[4];
-  __shared__ int wcnt[kPlanWaves][256];
-  __shared__ uint8_t sid8[LDS ? kPlanLdsRoutes : 1];
-  __shared__ uint16_t srank[LDS ? kPlanLdsRoutes : 1];
   const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = t >> 6;
   const int R = T * K;
+  const bool tiles = blockIdx.x + 1 == gridDim.x;
+  const int lo = tiles ? R : min((int)blockIdx.x * tokens_per_block, T) * K;
+  const int hi = tiles ? R : min(((int)blockIdx.x + 1) * tokens_per_block, T) * K;
   const unsigned long long lt = (1ull << lane) - 1ull;
-  auto load_eid = [&](int i) -> int {
+  auto eid = [&](int i) -> int {
     const int64_t e = ids[i];
     return (int)(e < 0 ? 0 : (e >= E ? E - 1 : e));
   };
-  auto eid = [&](int i) -> int {
-    if constexpr (LDS) return sid8[i];
-    else return load_eid(i);
-  };
-  auto rank_get = [&](int r) -> int {
-    if constexpr (LDS) return srank[r];
-    else return (int)ordered[r];
-  };
-  auto rank_set = [&](int r, int v) {
-    if constexpr (LDS) srank[r] = (uint16_t)v;
-    else ordered[r] = v;
-  };
-  if constexpr (LDS) {
-#pragma unroll 8
-    for (int r = t; r < R; r += kPlanThreads) sid8[r] = (uint8_t)load_eid(r);
-  }
-  if (t < 256)
-    for (int w = 0; w < kPlanWaves; ++w) wcnt[w][t] = 0;
+  for (int i = t; i < 512; i += kPlanThreads) count[i >> 8][i & 255] = 0;
+#pragma unroll
+  for (int i = 0; i < kPlanWaves * 256 / kPlanThreads; ++i)
+    wpos[(t + i * kPlanThreads) >> 8][t & 255] = 0;
   __syncthreads();
 
-  // Pass 1: rank of every route among equal ids of its wave's slice.
-  const int slice = ((R + kPlanWaves - 1) / kPlanWaves + 63) & ~63;
-  const int lo = wave * slice, hi = min(lo + slice, R);
-  for (int base = lo; base < hi; base += 64) {
+  // Counts: all routes, and per wave those of its own run.
+#pragma unroll 8
+  for (int r = t; r < R; r += kPlanThreads) atomicAdd(&count[r < lo ? 0 : 1][eid(r)], 1);
+  const int run = ((hi - lo + kPlanWaves - 1) / kPlanWaves + 63) & ~63;
+  const int wlo = min(lo + wave * run, hi), whi = min(wlo + run, hi);
+  for (int r = wlo + lane; r < whi; r += 64) atomicAdd(&wpos[wave][eid(r)], 1);
+  __syncthreads();
+  int all;
+  const int before = t < 256 ? count[0][t] : 0;
+  const int ex = block_scan_256(t < E ? before + count[1][t] : 0, scratch, &all);
+  if (t < 256) {
+    offs[t] = ex;
+    int p = ex + before;
+    for (int w = 0; w < kPlanWaves; ++w) {
+      const int c = wpos[w][t];
+      wpos[w][t] = p;
+      p += c;
+    }
+  }
+  if (t == 0) offs[256] = all;
+  __syncthreads();
+
+  // Sorted position p of each route of the slice, and its place i in its
+  // token: slots = argsort(ids, dim=1, stable), ordered[t, i] = p.
+  for (int base = wlo; base < whi; base += 64) {
     const int r = base + lane;
-    const bool valid = r < hi;
+    const bool valid = r < whi;
     const int e = valid ? eid(r) : 0;
     unsigned long long same = __ballot(valid);
 #pragma unroll
@@ -292,33 +287,25 @@ __global__ __launch_bounds__(1024) void route_plan_kernel(const int64_t *__restr
       same &= ((e >> b) & 1) ? bit : ~bit;
     }
     const int in_chunk = __popcll(same & lt);
-    const int before = valid ? wcnt[wave][e] : 0;
-    if (valid) rank_set(r, before + in_chunk);
-    if (valid && in_chunk == 0) wcnt[wave][e] = before + __popcll(same);
-  }
-  __syncthreads();
-  // Column scan: wcnt[w][e] becomes the count of e in slices before w.
-  int total_e = 0;
-  if (t < 256) {
-    for (int w = 0; w < kPlanWaves; ++w) {
-      const int c = wcnt[w][t];
-      wcnt[w][t] = total_e;
-      total_e += c;
+    const int first = wpos[wave][e];
+    wave_lds_sync();
+    if (valid && in_chunk == 0) wpos[wave][e] = first + __popcll(same);
+    wave_lds_sync();
+    if (valid) {
+      const int p = first + in_chunk;
+      const int tok = r / K, j = r - tok * K;
+      int i = 0;
+#pragma unroll 8
+      for (int jj = 0; jj < K; ++jj) {
+        const int o = eid(tok * K + jj);
+        i += (o < e || (o == e && jj < j)) ? 1 : 0;
+      }
+      pos[p] = tok;
+      slots[(int64_t)tok * K + i] = j;
+      ordered[(int64_t)tok * K + i] = p;
     }
   }
-  int all;
-  const int ex = block_scan_256(t < E ? total_e : 0, scratch, &all);
-  if (t < 256) offs[t] = ex;
-  if (t == 0) offs[256] = all;
-  __syncthreads();
-
-  // Pass 2: sorted position p of every route; pos[p] = its token.
-  for (int r = t; r < R; r += kPlanThreads) {
-    const int e = eid(r);
-    const int p = offs[e] + wcnt[r / slice][e] + rank_get(r);
-    pos[p] = r / K;
-    rank_set(r, p);
-  }
+  if (!tiles) return;
 
   // Tile table (gpu_routes._table): tiles of bm rows, expert by expert.
   const int nt = t < E ? (offs[t + 1] - offs[t] + bm - 1) / bm : 0;
@@ -344,57 +331,17 @@ __global__ __launch_bounds__(1024) void route_plan_kernel(const int64_t *__restr
     table[i * 3 + 1] = st_;
     table[i * 3 + 2] = sp_;
   }
-  // Always-on shared expert: its rows follow the R routed rows, gathered in
-  // token order, as extra tiles of expert E after the plan's max_tiles rows.
-  if (shared_rows > 0) {
-    const int nst = (shared_rows + bm - 1) / bm;
-    for (int j = t; j < nst; j += kPlanThreads) {
-      table[(int64_t)(max_tiles + j) * 3] = E;
-      table[(int64_t)(max_tiles + j) * 3 + 1] = R + (int64_t)j * bm;
-      table[(int64_t)(max_tiles + j) * 3 + 2] = R + shared_rows;
-    }
-    for (int tok = t; tok < shared_rows; tok += kPlanThreads) pos[R + tok] = tok;
-  }
-  __threadfence_block();
-  __syncthreads();
-
-  // slots = argsort(ids, dim=1, stable); ordered[t, i] = inverse[t*K + slots[t, i]].
-  auto token_order = [&](auto n_tag) {
-    constexpr int N = decltype(n_tag)::value;
-    for (int tok = t; tok < T; tok += kPlanThreads) {
-      int id[N], sl[N], iv[N];
-#pragma unroll
-      for (int j = 0; j < N; ++j) {
-        const bool in = j < K;
-        id[j] = in ? eid(tok * K + j) : 0x7FFFFFFF;
-        sl[j] = j;
-        iv[j] = in ? rank_get(tok * K + j) : 0;
-      }
-      sort_triples<N>(id, sl, iv);
-#pragma unroll
-      for (int j = 0; j < N; ++j) {
-        if (j < K) {
-          slots[(int64_t)tok * K + j] = sl[j];
-          ordered[(int64_t)tok * K + j] = iv[j];
-        }
-      }
-    }
-  };
-  if (K <= 8) token_order(std::integral_constant<int, 8>{});
-  else token_order(std::integral_constant<int, 16>{});
 }
 
 int route_plan(const int64_t *ids, int64_t T, int64_t K, int64_t E, int64_t bm, int64_t *pos,
                int64_t *table, int64_t max_tiles, int64_t *ordered, int64_t *slots,
-               int64_t shared_rows, hipStream_t st) {
-  if (T * K <= kPlanLdsRoutes)
-    route_plan_kernel<true><<<1, kPlanThreads, 0, st>>>(ids, (int)T, (int)K, (int)E, (int)bm, pos,
-                                                        table, (int)max_tiles, ordered, slots,
-                                                        (int)shared_rows);
-  else
-    route_plan_kernel<false><<<1, kPlanThreads, 0, st>>>(ids, (int)T, (int)K, (int)E, (int)bm,
-                                                         pos, table, (int)max_tiles, ordered,
-                                                         slots, (int)shared_rows);
+               hipStream_t st) {
+  const int64_t want = std::min<int64_t>((T * K + kPlanThreads - 1) / kPlanThreads, kPlanBlocks);
+  const int64_t per = (T + want - 1) / want;
+  const unsigned blocks = cdiv(T, per);
+  route_plan_kernel<<<blocks + 1, kPlanThreads, 0, st>>>(ids, (int)T, (int)K, (int)E, (int)bm,
+                                                         (int)per, pos, table, (int)max_tiles,
+                                                         ordered, slots);
   return check_launch("route_plan_kernel");
 }
 
@@ -525,7 +472,7 @@ extern "C" int lm_route_plan(const int64_t *ids, int64_t tokens, int64_t top_k, 
   LM_REQUIRE(max_tiles == (tokens * top_k + bm - 1) / bm + experts, LM_EINVAL,
              "max_tiles must be cdiv(routes, bm) + experts");
   LM_REQUIRE(ids && pos && table && ordered && slots, LM_EINVAL, "null pointer");
-  return route_plan(ids, tokens, top_k, experts, bm, pos, table, max_tiles, ordered, slots, 0,
+  return route_plan(ids, tokens, top_k, experts, bm, pos, table, max_tiles, ordered, slots,
                     as_stream(stream));
 }
 

@@ -358,6 +358,20 @@ def test_route_plan_bit_exact(dev, t, bm, skew):
         assert np.array_equal(g.cpu().numpy(), r), name
 
 
+@pytest.mark.parametrize('t,k,e,bm', [(129, 8, 256, 96), (257, 6, 200, 96), (1025, 1, 3, 64),
+                                      (700, 16, 40, 128), (40000, 8, 256, 96), (2049, 2, 1, 96)])
+def test_route_plan_slices(dev, t, k, e, bm):
+    """Calls of several slices, with ragged last slices, tokens that do not
+    divide a wave (k = 6), repeated ids within a token, one expert taking
+    every route, and slices of more than 1024 routes (40000 x 8)."""
+    g = np.random.default_rng(t + k)
+    ids = torch.from_numpy(np.minimum(g.integers(0, e, (t, k)), g.integers(0, e, (t, k))))
+    got = gpu_routes.plan(ids.to(dev), e, bm)
+    ref = O.plan(ids.numpy(), e, bm)
+    for a, r, name in zip(got, ref, ('pos', 'table', 'ordered', 'slots')):
+        assert np.array_equal(a.cpu().numpy(), r), name
+
+
 # ------------------------------------------------------------- a10/a13 routed GEMM
 @pytest.mark.parametrize('large', [False, True])
 def test_routed_gemm_exact_layout(dev, large):
