@@ -454,6 +454,27 @@ def test_routed_reduce_bit_exact(dev, dtype):
     assert torch.equal(y32, y)
 
 
+@pytest.mark.parametrize('k,n,off', [(1, 8, 0), (8, 2056, 0), (9, 1001, 0), (12, 520, 8), (8, 512, 3)])
+def test_routed_reduce_forms(dev, k, n, off):
+    """One to two batches of routes, rows that end inside a workgroup, odd
+    widths and misaligned rows (the one-column form): the same bits as the
+    oracle's combine."""
+    t, e = 7, 30
+    ids = _ids(seeded(k + n), t, e, k, False)
+    _, _, ordered, slots = gpu_routes.plan(ids.to(dev), e, 96)
+    gen = seeded(52)
+    v = (torch.randn(t * k, n, generator=gen) * 2).to(torch.bfloat16)
+    w = torch.softmax(torch.randn(t, k, generator=gen), -1).to(torch.bfloat16)
+    store = torch.empty(t * k * n + off, dtype=torch.bfloat16, device=dev)
+    vd = store[off:].view(t * k, n)
+    vd.copy_(v)
+    y = gpu_routes.routed_reduce(vd, ordered, slots, w.to(dev), t, n)
+    _, _, ro, rs = O.plan(ids.numpy(), e, 96)
+    for tok in range(t):
+        ref = O.ordered_combine(npf(v)[ro[tok]], npf(w)[tok, rs[tok]], O.bf16)
+        assert np.array_equal(npf(y[tok]), ref)
+
+
 LM_HEAD_N = 248320  # vocabulary of the 35B-A3B configuration
 
 
