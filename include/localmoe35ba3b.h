@@ -160,6 +160,38 @@ int lm_ordered_reduce(const void *v, const int64_t *table, const void *w,
                       int w_dtype, void *y, int64_t n, int64_t experts,
                       int dtype, void *stream);
 
+/* The descriptor table of the grouped decode GEMVs for n selected ids
+ * (ids_bytes 4 or 8: int32 or int64, clamped into [0, experts)):
+ * table[r, 5] = {gu_q + e * stride, gu_s + .., dn_q + .., dn_s + .., slot} of
+ * the r-th smallest id e (equal ids in selection order), slot its place in
+ * ids.  Strides in elements.  Replaces the host-built table of int8.py:164-179. */
+int lm_expert_table(const void *ids, int ids_bytes, int64_t n, int64_t experts,
+                    const int8_t *gu_q, const float *gu_s, const int8_t *dn_q,
+                    const float *dn_s, int64_t gu_q_expert_stride,
+                    int64_t gu_s_expert_stride, int64_t dn_q_expert_stride,
+                    int64_t dn_s_expert_stride, int64_t *table, void *stream);
+
+/* The W8A16 decode experts of one token in two launches: for the n selected
+ * ids in ascending order, h[r, :] = SwiGLU of x . gate_up[e]^T, then
+ * y = T(acc + T(T(h[r] . down[e]^T) * w[slot])) over r - the results of
+ * lm_w8a16_grouped_gemv, lm_swiglu, lm_w8a16_grouped_gemv and
+ * lm_ordered_reduce over lm_expert_table, bit for bit.  gate_up [2 * inter, hidden], down [hidden, inter] per
+ * expert; h [n, inter] is caller scratch in dtype; w [n] (w_dtype) by
+ * selection.  lm_w8a16_experts_decode_fits says whether (n, hidden, inter) is
+ * served (n <= 64 and the rows fit the workgroup's LDS); others take the
+ * separate calls.  Replaces the one-token path of Int8Experts.forward
+ * (int8.py:155-210). */
+int lm_w8a16_experts_decode_fits(int64_t n, int64_t hidden, int64_t inter);
+int lm_w8a16_experts_decode(const void *x, const void *ids, int ids_bytes,
+                            int64_t n, int64_t experts, const int8_t *gu_q,
+                            const float *gu_s, const int8_t *dn_q,
+                            const float *dn_s, int64_t gu_q_expert_stride,
+                            int64_t gu_s_expert_stride,
+                            int64_t dn_q_expert_stride,
+                            int64_t dn_s_expert_stride, const void *w,
+                            int w_dtype, void *h, void *y, int64_t hidden,
+                            int64_t inter, int dtype, void *stream);
+
 /* Prefill combine: per token over its top_k routes in ascending expert order
  * acc = T(acc + T(v[ordered[t,i], c] * w[t, slots[t,i]])), v and y of
  * `dtype` T; routes clamped into [0, tokens * top_k), slots into [0, top_k).

@@ -42,6 +42,10 @@ SIGNATURES = {
     'lm_w8a8_gemm': (I32, [P, P, P, P, P, I64, I64, I64, I32, I32, P]),
     'lm_swiglu': (I32, [P, P, I64, I64, I32, P]),
     'lm_ordered_reduce': (I32, [P, P, P, I32, P, I64, I64, I32, P]),
+    'lm_expert_table': (I32, [P, I32, I64, I64, P, P, P, P, I64, I64, I64, I64, P, P]),
+    'lm_w8a16_experts_decode_fits': (I32, [I64, I64, I64]),
+    'lm_w8a16_experts_decode': (I32, [P, P, I32, I64, I64, P, P, P, P, I64, I64, I64, I64, P, I32,
+                                      P, P, I64, I64, I32, P]),
     'lm_routed_reduce': (I32, [P, P, P, P, I32, P, I64, I64, I64, I32, P]),
     'lm_route_plan': (I32, [P, I64, I64, I64, I64, P, P, I64, P, P, P]),
     'lm_plan_routes_host': (I32, [P, I64, I64, I64, P, P, P, P, P]),

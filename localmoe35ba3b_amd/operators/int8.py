@@ -100,23 +100,37 @@ def swiglu(gu):
     return out
 
 
+def _selection(ids):
+    """The selected ids of one token as (flat contiguous tensor, element size)."""
+    if not ids.is_cuda or ids.dtype not in (torch.int64, torch.int32):
+        if not ids.is_cuda or ids.is_floating_point():
+            raise ValueError('Expected CUDA integer routing IDs')
+        ids = ids.to(torch.int64)
+    return ids.reshape(-1).contiguous(), ids.element_size()
+
+
+def _bank_args(gate_up, down):
+    gq, gs, dq, ds = gate_up['q'], gate_up['scale'], down['q'], down['scale']
+    return (gq.data_ptr(), gs.data_ptr(), dq.data_ptr(), ds.data_ptr(), gq.stride(0),
+            gs.stride(0), dq.stride(0), ds.stride(0))
+
+
 def build_descriptors(gate_up, down, ids):
     """Decode descriptor table for one token, sorted by expert id (int8.py:164-179).
 
     Returns a CUDA int64 [top_k, 5] table of (gate_up.q, gate_up.s, down.q,
     down.s) data pointers of each selected expert of the HBM bank plus its
-    slot, built on the device (no host read of the routing ids).
+    slot, built by one kernel (no host read of the routing ids).
     """
-    flat = ids.reshape(-1)
-    experts, slots = torch.sort(flat, stable=True)
-    bases = torch.tensor([gate_up['q'].data_ptr(), gate_up['scale'].data_ptr(),
-                          down['q'].data_ptr(), down['scale'].data_ptr()],
-                         dtype=torch.int64, device=ids.device)
-    strides = torch.tensor([gate_up['q'].stride(0), gate_up['scale'].stride(0) * 4,
-                            down['q'].stride(0), down['scale'].stride(0) * 4],
-                           dtype=torch.int64, device=ids.device)
-    ptrs = bases[None, :] + experts.to(torch.int64)[:, None] * strides[None, :]
-    return torch.cat([ptrs, slots.to(torch.int64)[:, None]], dim=1).contiguous()
+    flat, size = _selection(ids)
+    n = flat.numel()
+    table = torch.empty((n, 5), dtype=torch.int64, device=flat.device)
+    _lib.call('lm_expert_table', flat.data_ptr(), size, n, gate_up['q'].shape[0],
+              *_bank_args(gate_up, down), table.data_ptr(), _lib.stream(flat.device))
+    return table
+
+
+_w8a16_grouped_linear = grouped_linear  # the operator the two-launch decode computes
 
 
 class Int8Experts(torch.nn.Module):
@@ -130,7 +144,8 @@ class Int8Experts(torch.nn.Module):
         device-planned routed MoE (gpu_routes.routed_moe);
       * M == 1: grouped decode - module-level grouped_linear (W8A16, or W8A8
         after `int8.grouped_linear = w8a8.grouped_linear`), SwiGLU, and the
-        ordered bf16 combine in ascending expert order.
+        ordered bf16 combine in ascending expert order; while grouped_linear
+        is the W8A16 operator, in two fused launches with the same results.
     """
 
     def __init__(self, layer, gate_up, down, cache=None):
@@ -150,10 +165,31 @@ class Int8Experts(torch.nn.Module):
             banks = [self.gate_up['q'], self.gate_up['scale'], self.down['q'], self.down['scale']]
             return gpu_routes.routed_moe(x, top_k_weights, top_k_index.contiguous(), banks,
                                          self.large_tile)
+        hidden, intermediate = x.shape[-1], self.down['q'].shape[-1]
+        if (grouped_linear is _w8a16_grouped_linear
+                and _lib.lib().lm_w8a16_experts_decode_fits(top_k_index.numel(), hidden,
+                                                            intermediate)):
+            return self._decode(x, top_k_index, top_k_weights, hidden, intermediate)
         table = build_descriptors(self.gate_up, self.down, top_k_index)
         experts = table.shape[0]
-        intermediate = self.down['q'].shape[-1]
         gu = grouped_linear(x, table, experts, 2 * intermediate, 0, True)
         h = swiglu(gu)
-        values = grouped_linear(h, table, experts, x.shape[-1], 2, False)
+        values = grouped_linear(h, table, experts, hidden, 2, False)
         return ordered_reduce(values, table, top_k_weights)
+
+    def _decode(self, x, ids, weights, hidden, intermediate):
+        """One token, W8A16: gate_up + SwiGLU, then down + combine, two launches
+        with the results of the separate operators."""
+        if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16):
+            raise ValueError('W8A16 requires CUDA FP16/BF16 activations')
+        x, weights = x.contiguous(), weights.contiguous()
+        flat, size = _selection(ids)
+        n = flat.numel()
+        h = torch.empty((n, intermediate), dtype=x.dtype, device=x.device)
+        out = torch.empty((1, hidden), dtype=x.dtype, device=x.device)
+        _lib.call('lm_w8a16_experts_decode', x.data_ptr(), flat.data_ptr(), size, n,
+                  self.gate_up['q'].shape[0], *_bank_args(self.gate_up, self.down),
+                  weights.data_ptr(), _lib.dtype_code(weights.dtype), h.data_ptr(),
+                  out.data_ptr(), hidden, intermediate, _lib.dtype_code(x.dtype),
+                  _lib.stream(x.device))
+        return out

@@ -252,6 +252,36 @@ def test_w8a16_grouped_and_experts_decode(dev):
     assert_close(npf(out8)[0], O.ordered_combine(vals8, wsorted), BF16_TOL, 'Int8Experts w8a8')
 
 
+@pytest.mark.parametrize('n,hidden,inter,dtype,idt', [
+    (8, 2048, 512, torch.bfloat16, torch.int64), (1, 2048, 512, torch.float16, torch.int64),
+    (3, 2048, 384, torch.bfloat16, torch.int32), (9, 2048, 512, torch.float16, torch.int64),
+    (12, 1024, 512, torch.bfloat16, torch.int64), (40, 384, 640, torch.bfloat16, torch.int64),
+    (70, 256, 128, torch.bfloat16, torch.int64)])
+def test_experts_decode_forms(dev, n, hidden, inter, dtype, idt):
+    """One token through Int8Experts against the separate operators, bit for
+    bit: one to several batches of rows, widths other than the model's,
+    repeated ids, and more experts than the fused launches serve (70)."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(n + inter)
+    e = 11
+    bank = [convert.quantize_g128(torch.randn(e, a, b, generator=g, device=dev) * 0.02)
+            for a, b in ((2 * inter, hidden), (hidden, inter))]
+    (gq, gs), (dq, ds) = bank
+    gate_up, down = {'q': gq, 'scale': gs}, {'q': dq, 'scale': ds}
+    ids = torch.randint(0, e, (1, n), generator=g, device=dev).to(idt)
+    wts = torch.rand(1, n, generator=g, device=dev).to(dtype)
+    x = torch.randn(1, hidden, generator=g, device=dev).to(dtype)
+    out = int8.Int8Experts(0, gate_up, down)(x, ids, wts)
+    table = int8.build_descriptors(gate_up, down, ids)
+    order = torch.sort(ids.reshape(-1).long(), stable=True)
+    assert torch.equal(table[:, 4], order.indices)
+    for c, (t, size) in enumerate(((gq, 1), (gs, 4), (dq, 1), (ds, 4))):
+        assert torch.equal(table[:, c], t.data_ptr() + order.values * t.stride(0) * size)
+    h = int8.swiglu(int8.grouped_linear(x, table, n, 2 * inter, 0, True))
+    ref = int8.ordered_reduce(int8.grouped_linear(h, table, n, hidden, 2, False), table, wts)
+    assert torch.equal(out, ref)
+
+
 # ------------------------------------------------------------- a6/a11/a12 glue
 def test_ordered_reduce_bit_exact(dev):
     gen = seeded(7)
