@@ -125,6 +125,24 @@ __device__ __forceinline__ u32x4 dequant8s(uint2 w, float s) {
                T::pack2(f[6], f[7])};
 }
 
+// Eight weights of the LM_TILES_F16 format (bytes u = q + 128, each dword
+// holding k = 0, 2, 1, 3 in byte order) -> eight fp16 values q, exactly, in k
+// order.  A byte placed under the fp16 exponent of 1024 is the value 1024 + u
+// (one v_bitop3 (S0 & S1) | S2 for k = 0, 1, one byte permute for k = 2, 3);
+// subtracting 1152 leaves q.  Four VALU operations per four weights, against
+// eleven for the exact bf16(q * s).
+__device__ __forceinline__ u32x4 dequant8_f16(uint2 w) {
+  constexpr unsigned kAndOr = (0xF0u & 0xCCu) | 0xAAu;  // bitop3 table of (S0 & S1) | S2
+  const f16x2 bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+  auto sub = [&](uint32_t m) {
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, m) + bias);
+  };
+  return u32x4{sub(__builtin_amdgcn_bitop3_b32(w.x, 0x00FF00FFu, 0x64006400u, kAndOr)),
+               sub(__builtin_amdgcn_perm(0x64646464u, w.x, 0x07030701u)),
+               sub(__builtin_amdgcn_bitop3_b32(w.y, 0x00FF00FFu, 0x64006400u, kAndOr)),
+               sub(__builtin_amdgcn_perm(0x64646464u, w.y, 0x07030701u))};
+}
+
 // ------------------------------------------------------------ lane reductions
 // Sums over the 8 lanes of each lane octet (lanes 8j..8j+7); every lane of the
 // octet receives the total.  DPP: xor-1 and xor-2 quad permutations, then the
@@ -233,6 +251,12 @@ __device__ __forceinline__ float add_rn(float a, float b) { return a + b; }
 
 __device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + expf(-x)); }
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+// SiLU for the prefill epilogue from the hardware exp2 and reciprocal
+// (about 2 ulp in fp32); the product is rounded to bf16 right after.
+__device__ __forceinline__ float silu_fast(float x) {
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
+}
 
 // Order-preserving keys packing a logit with an index so that larger key =
 // (larger value, then smaller index); -0 is folded onto +0 and comes back as

@@ -58,6 +58,7 @@ struct GemmArgs {
   int tile_rows;  // rows covered by one table tile (<= BM)
   int nt_count;   // column tiles
   int mt_count;   // row tiles (table rows, or dense M tiles)
+  bool few_rows;     // routed: few rows per expert on average (kFewRows)
   bool cols_by_xcd;  // dense: a column tile's row tiles share an XCD, not a row tile's columns
 };
 
@@ -266,30 +267,6 @@ __global__ __launch_bounds__(256) void w8a16_mfma_kernel(GemmArgs a) {
 // are prefetched into registers while the current stage computes.
 constexpr int kGBM = 128;
 constexpr int kLDB = kBK + 8;  // int8 bytes per LDS row of the weight tile
-
-// Eight weights of the LM_TILES_F16 format (bytes u = q + 128, each dword
-// holding k = 0, 2, 1, 3 in byte order) -> eight fp16 values q, exactly, in k
-// order.  A byte placed under the fp16 exponent of 1024 is the value 1024 + u
-// (one v_bitop3 (S0 & S1) | S2 for k = 0, 1, one byte permute for k = 2, 3);
-// subtracting 1152 leaves q.  Four VALU operations per four weights, against
-// eleven for the exact bf16(q * s).
-__device__ __forceinline__ u32x4 dequant8_f16(uint2 w) {
-  constexpr unsigned kAndOr = (0xF0u & 0xCCu) | 0xAAu;  // bitop3 table of (S0 & S1) | S2
-  const f16x2 bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-  auto sub = [&](uint32_t m) {
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, m) + bias);
-  };
-  return u32x4{sub(__builtin_amdgcn_bitop3_b32(w.x, 0x00FF00FFu, 0x64006400u, kAndOr)),
-               sub(__builtin_amdgcn_perm(0x64646464u, w.x, 0x07030701u)),
-               sub(__builtin_amdgcn_bitop3_b32(w.y, 0x00FF00FFu, 0x64006400u, kAndOr)),
-               sub(__builtin_amdgcn_perm(0x64646464u, w.y, 0x07030701u))};
-}
-
-// SiLU for the prefill epilogue from the hardware exp2 and reciprocal
-// (about 2 ulp in fp32); the product is rounded to bf16 right after.
-__device__ __forceinline__ float silu_fast(float x) {
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
-}
 
 template <typename T>
 __device__ __forceinline__ u32x4 dequant8(uint2 w, float s) {
@@ -868,8 +845,11 @@ __device__ __forceinline__ void rb_tile(const GemmArgs &a, int64_t e, int64_t st
   }
 }
 
+// DEEP: tiles of at most 32 rows (64 rows) run a 5-slot (4-slot) weight ring
+// and 3-stage activations: their few accumulators leave the registers, and a
+// tile that computes little lives on the weight stages it has in flight.
 template <typename T, bool SWIGLU, bool GATHER, int WL, int K, int BM, int TN, int BD, int HL,
-          int AD, int NW, int OCC>
+          int AD, int NW, int OCC, bool DEEP>
 __global__ __launch_bounds__(NW * 64, OCC) void grouped_rb_kernel(GemmArgs a) {
   constexpr int SC_BYTES = NW * TN * (K / 128) * 4 + (WL == kWlTilesF16 ? (NW * TN + BM) * 4 : 0);
   __shared__ __align__(16) unsigned char smem[3 * BM * 128 * HL + SC_BYTES];
@@ -919,14 +899,17 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_rb_kernel(GemmArgs a) {
       rb_tile<T, SWIGLU, GATHER, WL, K, BM, TN, BD, HL, AD, NW, 2>(a, e, start, rows, nt, smem, gx, gk);
   } else {
     static_assert(BM == 96, "row-count dispatch below covers 96-row tiles");
+    constexpr int BDS = DEEP ? 5 : BD, ADS = DEEP ? 3 : AD, BDM = DEEP ? 4 : BD;
     if (rows > 80)
       rb_tile<T, SWIGLU, GATHER, WL, K, BM, TN, BD, HL, AD, NW, 6>(a, e, start, rows, nt, smem, gx, gk);
     else if (rows > 64)
       rb_tile<T, SWIGLU, GATHER, WL, K, BM, TN, BD, HL, AD, NW, 5>(a, e, start, rows, nt, smem, gx, gk);
     else if (rows > 32)
-      rb_tile<T, SWIGLU, GATHER, WL, K, BM, TN, BD, HL, AD, NW, 4>(a, e, start, rows, nt, smem, gx, gk);
+      rb_tile<T, SWIGLU, GATHER, WL, K, BM, TN, BDM, HL, AD, NW, 4>(a, e, start, rows, nt, smem, gx, gk);
+    else if (!DEEP || rows > 16)
+      rb_tile<T, SWIGLU, GATHER, WL, K, BM, TN, BDS, HL, ADS, NW, 2>(a, e, start, rows, nt, smem, gx, gk);
     else
-      rb_tile<T, SWIGLU, GATHER, WL, K, BM, TN, BD, HL, AD, NW, 2>(a, e, start, rows, nt, smem, gx, gk);
+      rb_tile<T, SWIGLU, GATHER, WL, K, BM, TN, BDS, HL, ADS, NW, 1>(a, e, start, rows, nt, smem, gx, gk);
   }
 }
 
@@ -958,6 +941,12 @@ constexpr int kGroupedBN = 128;  // grouped_mfma_kernel tile columns
 constexpr int kRbBMTall = 128;
 constexpr int kRbADTall = 3;
 constexpr int64_t kDenseTallM = 1024;
+// Few rows per expert (a short prompt, a small batch): gate_up on the tile
+// layout takes 32 columns per wave at 3 workgroups per CU and the deep rings
+// instead: 26 -> 17 us at 2 tokens, 66 -> 53 at 24, 110 -> 95 at 256, 117 ->
+// 111 at 1024 (256 experts, top-8).  Above that a chunk overlaps with another one,
+// where the 64-column form is faster (above).
+constexpr int64_t kFewRows = 36;
 // Wide dense tiles: 8 waves over 256 columns of a 128-row tile, one
 // workgroup per CU.  Each activation stage then feeds twice the columns, a
 // third fewer wave-loads per MFMA than two 4-wave workgroups; taken when the
@@ -965,22 +954,26 @@ constexpr int64_t kDenseTallM = 1024;
 constexpr int kRbNWWide = 8;
 constexpr int64_t kRbWideTiles = 256;
 
-template <typename T, bool SWIGLU, bool GATHER, int WL, int K, int BM = 96, int NW = kRbNW>
+template <typename T, bool SWIGLU, bool GATHER, int WL, int K, int BM = 96, int NW = kRbNW,
+          bool FEW = false>
 static int launch_rb(GemmArgs a, unsigned mtiles, hipStream_t st) {
-  constexpr bool TILES = WL == kWlTiles || WL == kWlTilesF16;
+  constexpr bool TILES = (WL == kWlTiles || WL == kWlTilesF16) && !FEW;  // the 64-column form
   constexpr bool TALL = BM == kRbBMTall;
   static_assert(!TALL || (WL == kWlDirect && !SWIGLU && !GATHER), "tall tiles serve dense rows");
   static_assert(NW == kRbNW || (TALL && NW == kRbNWWide), "wide tiles serve dense tall rows");
   constexpr int TN = TILES ? kRbTnTiles : kRbTN;
   constexpr int OCC = NW == kRbNWWide ? 1 : TILES || TALL ? kRbOccTiles : kRbOcc;
   constexpr int AD = TALL ? kRbADTall : kRbAD;
+  // gate_up at 32 columns per wave; the down GEMM's 8 stages are no longer
+  // than the deep ring, which made it slower (33 -> 39 us at 24 tokens)
+  constexpr bool DEEP = K == 2048 && WL != kWlDirect && TN == kRbTN;
   constexpr int RBN = NW * TN;
   a.nt_count = SWIGLU ? (int)cdiv(a.N / 2, RBN / 2) : (int)cdiv(a.N, RBN);
   a.mt_count = (int)mtiles;
   const int64_t grid = xcd_grid(a.mt_count, a.nt_count, a.cols_by_xcd);
   LM_REQUIRE(grid < (int64_t(1) << 31), LM_EINVAL, "problem too large for one launch");
-  grouped_rb_kernel<T, SWIGLU, GATHER, WL, K, BM, TN, kRbBD, kRbHL, AD, NW, OCC>
-      <<<(unsigned)grid, NW * 64, 0, st>>>(a);
+  grouped_rb_kernel<T, SWIGLU, GATHER, WL, K, BM, TN, kRbBD, kRbHL, AD, NW, OCC,
+                    DEEP><<<(unsigned)grid, NW * 64, 0, st>>>(a);
   return check_launch("grouped_rb_kernel");
 }
 
@@ -1002,6 +995,10 @@ static int launch_grouped(GemmArgs a, unsigned mtiles, hipStream_t st) {
       if (a.K == 2048) return go(std::integral_constant<int, 2048>{});
       return go(std::integral_constant<int, 512>{});
     }
+  }
+  if constexpr (SWIGLU && (WL == kWlTiles || WL == kWlTilesF16)) {
+    if (a.few_rows && a.K == 2048)
+      return launch_rb<T, SWIGLU, GATHER, WL, 2048, 96, kRbNW, true>(a, mtiles, st);
   }
   if (a.tile_rows <= 96 && (a.K == 2048 || a.K == 512))
     return a.K == 2048 ? launch_rb<T, SWIGLU, GATHER, WL, 2048>(a, mtiles, st)
@@ -1125,6 +1122,7 @@ int routed_gemm(const RoutedGemm &r, hipStream_t st) {
   a.N = (int)r.n;
   a.K = (int)r.k;
   a.tile_rows = (int)r.bm;
+  a.few_rows = r.y_rows <= kFewRows * r.experts;
   const unsigned mt = (unsigned)r.n_tiles;
   return r.dtype == LM_BF16 ? routed_dispatch<BF16>(a, mt, r.gather, r.swiglu, st)
                             : routed_dispatch<FP16>(a, mt, r.gather, r.swiglu, st);

@@ -1076,6 +1076,8 @@ __global__ __launch_bounds__(kTopkTokens * 64) void prefill_topk_count_kernel(
       e = (int)clamp_index(sid[w][lane], kE);
       a.ids[(int64_t)tok * kTopK + lane] = e;
       a.wts[(int64_t)tok * kTopK + lane] = swt[w][lane];
+      if (a.ids_out) a.ids_out[(int64_t)tok * kTopK + lane] = e;
+      if (a.wts_out) a.wts_out[(int64_t)tok * kTopK + lane] = swt[w][lane];
       rank = atomicAdd(&lcnt[e], 1);
     }
   }
@@ -1325,14 +1327,6 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(int64_t *p_ids, co
     prefill_norm_token(outv, nwv, gv, b, tok, red, red2, dred);
     if (tok < kE) router_row_norm(wv, a.nw + tok, red2);
   }
-}
-
-__global__ void export_routing_kernel(const int64_t *ids, const uint16_t *wts, int32_t *ids_out,
-                                      uint16_t *wts_out, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  if (ids_out) ids_out[i] = (int32_t)ids[i];
-  if (wts_out) wts_out[i] = wts[i];
 }
 
 // Zeroes n bytes (n a multiple of 4) with a grid-stride loop of dword stores.
@@ -1645,12 +1639,7 @@ int layer_forward(const lm_moe_layer *layer, const lm_moe_layer *next, bool inpu
                                                               a, NextLayer{});
   }
   if (int rc = check_launch("prefill_combine_kernel")) return rc;
-  if (int rc = mark(7)) return rc;
-  if (ids_out || weights_out) {
-    export_routing_kernel<<<cdiv(R, 256), 256, 0, st>>>(a.ids, a.wts, ids_out, a.wts_out, R);
-    return check_launch("export_routing_kernel");
-  }
-  return LM_OK;
+  return mark(7);
 }
 }  // namespace
 

@@ -330,6 +330,22 @@ def test_prefill_extreme_inputs(dev, fmt, monkeypatch):
 
 
 @pytest.mark.parametrize('fmt', [0, 1])
+@pytest.mark.parametrize('tokens', [2, 37, 300, 1027])
+def test_few_row_tiles(dev, fmt, tokens):
+    """The gate_up form of few rows per expert (32 columns per wave, up to
+    1027 tokens) against the 64-column form of a larger call: each token's
+    result is the same bits in both.  The Zipf routing gives tiles of every row
+    count from 1 to 96 (the deep rings up to 32 and 64 rows, and the full tiles)."""
+    st = SyntheticMoEStack(layers=1, seed=41, device=dev, max_tokens=1600,
+                           router_bias=zipf_bias(), gate_up_format=fmt)
+    x = inputs(1600, 42, dev)
+    whole, ids, wts = run_layer(st, x)
+    part, pids, pwts = run_layer(st, x[:tokens].contiguous())
+    assert torch.equal(pids, ids[:tokens]) and torch.equal(pwts, wts[:tokens])
+    assert torch.equal(part, whole[:tokens])
+
+
+@pytest.mark.parametrize('fmt', [0, 1])
 @pytest.mark.parametrize('tokens', [1, 100, 300])
 def test_chained_layers_bit_identical(dev, fmt, tokens):
     """Chained layer calls (lm_moe_layer_forward_chain: each combine does the
