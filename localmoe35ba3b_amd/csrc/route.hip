@@ -64,81 +64,97 @@ __global__ __launch_bounds__(256) void router_logits_gemv(const uint16_t *__rest
   }
 }
 
-// Large token counts (prefill): v_mfma_f64_16x16x4f64.  Block = 4 waves,
-// tile 16 tokens x 128 experts, each wave 16 x 32.  Lane quad q supplies
-// k = k0 + 8 q + j at MFMA step j (the same permutation for both operands),
-// so one 16-byte load per operand row feeds 8 MFMA steps.
-template <int D>
-__global__ __launch_bounds__(256) void router_logits_mfma(const uint16_t *__restrict__ x,
-                                                          const uint16_t *__restrict__ w,
-                                                          const float *__restrict__ bias,
-                                                          float *__restrict__ logits, int T,
-                                                          int E, int H) {
-  // One wave = 16 tokens x 32 experts; K in 32-wide stages held in a
-  // D-stage register ring (D - 1 stages in flight while one is consumed;
-  // H must be a multiple of 32 D).  Even and odd K-steps accumulate into
-  // separate fp64 tiles, added at the end, so four independent MFMA chains
-  // are in flight.
+// More tokens: v_mfma_f64_16x16x4f64.  A workgroup owns 16 tokens x 16 NE
+// experts and its waves split K (K in 32-wide stages dealt round robin, so any
+// number of stages splits evenly); the fp64 partial tiles are added through
+// LDS.  Lane quad q supplies k = k0 + 8 q + j at MFMA step j (the same
+// permutation for both operands), so one 16-byte load per operand row feeds 8
+// MFMA steps.  Two stages are held in registers, and even and odd K-steps
+// accumulate into separate fp64 tiles.
+//
+// Bound: the fp64 matrix rate (64 cycles per MFMA and SIMD: 27 us for 2048
+// tokens x 256 experts x 2048; 7 us for one 16 x 32 tile on a CU).  With all of
+// K in one wave and 32 x 128 experts per workgroup a call of 9 tokens took as
+// long as one of 2048 (46 us, top-k included); split it takes 12 us up to 256
+// tokens, 17 up to 512, 27 up to 1024 and 45 at 2048.
+constexpr int kRouterWaves = 4;
+template <int NE>
+__global__ __launch_bounds__(kRouterWaves * 64) void router_logits_mfma(
+    const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, const float *__restrict__ bias,
+    float *__restrict__ logits, int T, int E, int H) {
+  constexpr int NW = kRouterWaves, D = 2;
+  __shared__ f64x4 part[NW][NE][64];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int t0 = blockIdx.x * 16;
-  const int e0 = blockIdx.y * 128 + wave * 32;
-  if (e0 >= E) return;
+  const int e0 = blockIdx.y * 16 * NE;
   const int q = lane >> 4;
   const int r = lane & 15;
   const uint16_t *xa = x + (int64_t)min(t0 + r, T - 1) * H + q * 8;
-  const uint16_t *wb0 = w + (int64_t)min(e0 + r, E - 1) * H + q * 8;
-  const uint16_t *wb1 = w + (int64_t)min(e0 + 16 + r, E - 1) * H + q * 8;
-  f64x4 acc[2][2] = {{{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}},
-                     {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}}};
-  u32x4 ra[D], rb0[D], rb1[D];
-  const int last = H - 32;
+  const uint16_t *wb[NE];
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    const int k = min(32 * d, last);
-    ra[d] = ldg16(xa + k);
-    rb0[d] = ldg16(wb0 + k);
-    rb1[d] = ldg16(wb1 + k);
-  }
-  for (int k0 = 0; k0 < H; k0 += 32 * D) {
+  for (int c = 0; c < NE; ++c) wb[c] = w + (int64_t)min(e0 + 16 * c + r, E - 1) * H + q * 8;
+  f64x4 acc[2][NE];
 #pragma unroll
-    for (int u = 0; u < D; ++u) {
-      const u32x4 av = ra[u], bv0 = rb0[u], bv1 = rb1[u];
-      // refill the slot with the stage D ahead (clamped: past the end the
-      // last stage is re-read and never consumed)
-      const int kn = min(k0 + 32 * (u + D), last);
-      ra[u] = ldg16(xa + kn);
-      rb0[u] = ldg16(wb0 + kn);
-      rb1[u] = ldg16(wb1 + kn);
+  for (int c = 0; c < NE; ++c) acc[0][c] = acc[1][c] = f64x4{0.0, 0.0, 0.0, 0.0};
+  u32x4 ra[D], rb[D][NE];
+  // this wave's stages: k = 32 (NW i + wave), i < stages; past the end the
+  // row's last stage is re-read and never consumed
+  const int stages = (H / 32 - wave + NW - 1) / NW;
+  auto load = [&](int slot, int i) {
+    const int k = min(32 * (NW * i + wave), H - 32);
+    ra[slot] = ldg16(xa + k);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t sh = (j & 1) ? 16u : 0u;
-        const double a = (double)bf16_bits_to_f32((av[j >> 1] >> sh) & 0xFFFFu);
-        const double b0 = (double)bf16_bits_to_f32((bv0[j >> 1] >> sh) & 0xFFFFu);
-        const double b1 = (double)bf16_bits_to_f32((bv1[j >> 1] >> sh) & 0xFFFFu);
-        acc[j & 1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b0, acc[j & 1][0], 0, 0, 0);
-        acc[j & 1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b1, acc[j & 1][1], 0, 0, 0);
+    for (int c = 0; c < NE; ++c) rb[slot][c] = ldg16(wb[c] + k);
+  };
+  auto step = [&](u32x4 av, const u32x4 (&bv)[NE]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t sh = (j & 1) ? 16u : 0u;
+      const double a = (double)bf16_bits_to_f32((av[j >> 1] >> sh) & 0xFFFFu);
+#pragma unroll
+      for (int c = 0; c < NE; ++c) {
+        const double b = (double)bf16_bits_to_f32((bv[c][j >> 1] >> sh) & 0xFFFFu);
+        acc[j & 1][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[j & 1][c], 0, 0, 0);
       }
     }
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d);
+  int i = 0;
+  for (; i + D <= stages; i += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      const u32x4 av = ra[u];
+      u32x4 bv[NE];
+#pragma unroll
+      for (int c = 0; c < NE; ++c) bv[c] = rb[u][c];
+      load(u, i + u + D);
+      step(av, bv);
+    }
   }
+#pragma unroll
+  for (int u = 0; u < D; ++u)
+    if (i + u < stages) step(ra[u], rb[u]);
+#pragma unroll
+  for (int c = 0; c < NE; ++c) part[wave][c][lane] = acc[0][c] + acc[1][c];
+  __syncthreads();
+  if (wave >= NE) return;  // wave c finishes 16 experts
+  f64x4 v = part[0][wave][lane];
+#pragma unroll
+  for (int j = 1; j < NW; ++j) v = v + part[j][wave][lane];
   // D layout of the f64 16x16x4 MFMA: lane holds column (lane & 15) and
   // rows (lane >> 4) + 4 i, i = 0..3 (unlike the 4 (lane >> 4) + i rows of the
   // 32-bit-output 16x16 MFMAs).
+  const int e = e0 + 16 * wave + r;
+  if (e >= E) return;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int t = t0 + q + 4 * i;
+  for (int m = 0; m < 4; ++m) {
+    const int t = t0 + q + 4 * m;
     if (t >= T) continue;
-    const int ea = e0 + r, eb = e0 + 16 + r;
-    if (ea < E) {
-      float l = round_bf16((float)(acc[0][0][i] + acc[1][0][i]));
-      if (bias) l = l + bias[ea];
-      logits[(int64_t)t * E + ea] = l;
-    }
-    if (eb < E) {
-      float l = round_bf16((float)(acc[0][1][i] + acc[1][1][i]));
-      if (bias) l = l + bias[eb];
-      logits[(int64_t)t * E + eb] = l;
-    }
+    float l = round_bf16((float)v[m]);
+    if (bias) l = l + bias[e];
+    logits[(int64_t)t * E + e] = l;
   }
 }
 
@@ -156,18 +172,18 @@ __global__ __launch_bounds__(256) void topk_kernel(const float *__restrict__ log
 
 int router_logits(const uint16_t *x, const uint16_t *w, const float *bias, float *logits,
                   int64_t T, int64_t E, int64_t H, hipStream_t st) {
-  if (T <= 8) {
+  if (T <= 6) {  // 11.5 us and rising with T; the MFMA tile takes 12
     const unsigned g = cdiv(E, 4);
     if (T == 1)
       router_logits_gemv<1><<<g, 256, 0, st>>>(x, w, bias, logits, (int)T, (int)E, (int)H);
     else
       router_logits_gemv<8><<<g, 256, 0, st>>>(x, w, bias, logits, (int)T, (int)E, (int)H);
+  } else if (cdiv(T, 16) * cdiv(E, 16) <= 256) {  // narrow tiles while they fit the CUs once
+    router_logits_mfma<1><<<dim3(cdiv(T, 16), cdiv(E, 16)), kRouterWaves * 64, 0, st>>>(
+        x, w, bias, logits, (int)T, (int)E, (int)H);
   } else {
-    const dim3 grid(cdiv(T, 16), cdiv(E, 128));
-    if (H % 128 == 0)
-      router_logits_mfma<4><<<grid, 256, 0, st>>>(x, w, bias, logits, (int)T, (int)E, (int)H);
-    else
-      router_logits_mfma<1><<<grid, 256, 0, st>>>(x, w, bias, logits, (int)T, (int)E, (int)H);
+    router_logits_mfma<2><<<dim3(cdiv(T, 16), cdiv(E, 32)), kRouterWaves * 64, 0, st>>>(
+        x, w, bias, logits, (int)T, (int)E, (int)H);
   }
   return check_launch("router_logits");
 }

@@ -361,6 +361,23 @@ def test_router_key_widths(dev, bias_kind):
     assert ids[5].cpu().tolist() == ri[5].tolist()
 
 
+@pytest.mark.parametrize('t,e,h,k', [(6, 256, 2048, 8), (7, 33, 96, 8), (16, 16, 32, 4),
+                                     (17, 250, 2080, 16), (256, 256, 160, 8), (257, 256, 64, 8),
+                                     (700, 200, 224, 2)])
+def test_router_shapes(dev, t, e, h, k):
+    """The router's row and expert tiles at their edges (16 x 16 and 16 x 32),
+    K stages that do not divide over the waves (1, 2, 3, 5, 7 and 65 of them):
+    logits and ids equal the oracle's."""
+    gen = seeded(t + e)
+    x = bf16_rand((t, h), gen)
+    w = bf16_rand((e, h), gen, 0.05)
+    lg, wts, ids = router.router_topk(x.to(dev), w.to(dev), k)
+    rl, rw, ri = O.router(npf(x), npf(w), k)
+    assert np.array_equal(lg.cpu().numpy(), rl)
+    assert np.array_equal(ids.cpu().numpy(), ri)
+    assert np.abs(npf(wts) - rw).max() <= 2.0 ** -8
+
+
 def test_rmsnorm_bit_exact(dev):
     gen = seeded(11)
     x = bf16_rand((5, 2048), gen, 3.0)
