@@ -1,6 +1,7 @@
 // Decode GEMV kernels behind the generic operator entry points:
 //   lm_w8a8_grouped_gemv / lm_w8a8_grouped_linear   (w8a8.py:25-48)
 //   lm_w8a8_linear (dense, optional SwiGLU)          (config: W8A8 gate_up)
+//   lm_w8a8_gemm for m <= 16 at K = 2048             (w8a8_gemv_rows)
 //   lm_w8a8_group_partials                           (exact int32 partials)
 //   lm_w8a16_grouped_gemv                            (int8.py:213-237)
 //   lm_w8a16_linear for m <= 8                       (int8.py:9-37)
@@ -342,6 +343,11 @@ static int launch_w8a8(const GemvArgs &a, unsigned gy, hipStream_t st) {
   LM_REQUIRE(lds <= 160 * 1024, LM_EINVAL, "Invalid INT8 group geometry");
   const unsigned gx = a.swiglu ? cdiv(a.N / 2, a.RB / 2) : cdiv(a.N, a.RB);
   const dim3 grid(gx, gy);
+  if constexpr (MT > 8) {  // w8a8_gemv_rows: K = 2048
+    w8a8_gemv_kernel<T, MT, QUANT, PARTIALS, 2048, kGemvThreadsK>
+        <<<grid, kGemvThreadsK, lds, st>>>(a);
+    return check_launch("w8a8_gemv_kernel");
+  }
   const bool large = gemv_large_blocks((int64_t)gx * gy, MT);
   if (a.K == 2048 && large)
     w8a8_gemv_kernel<T, MT, QUANT, PARTIALS, 2048, kGemvThreadsK>
@@ -408,6 +414,31 @@ static int dispatch_w8a16(const GemvArgs &a, unsigned gy, hipStream_t st) {
     case 4: return launch_w8a16<T, 4>(a, gy, st);
     default: return launch_w8a16<T, 8>(a, gy, st);
   }
+}
+
+// Up to 16 rows already quantized, K = 2048: the GEMV's K-parallel MFMA form,
+// whose epilogue adds the groups in the GEMM's order (5.0 to 5.8 us at N = 512
+// to 4096, where the GEMM's smallest tile, walking K alone, takes 8.5; at K =
+// 512 the tile is as fast, and with 32 rows this form spills).
+bool w8a8_gemv_serves(int64_t m, int64_t k) { return m <= 16 && k == 2048; }
+
+int w8a8_gemv_rows(const int8_t *xq, const float *xs, const int8_t *q, const float *s, void *y,
+                   int64_t m, int64_t n, int64_t k, int swiglu, int y_dtype, hipStream_t st) {
+  GemvArgs a{};
+  a.q = q;
+  a.s = s;
+  a.xq = xq;
+  a.xs = xs;
+  a.M = (int)m;
+  a.y = static_cast<uint16_t *>(y);
+  a.ldy = swiglu ? n / 2 : n;
+  a.N = (int)n;
+  a.K = (int)k;
+  a.RB = gemv_rows_per_block(k);
+  a.swiglu = swiglu ? 1 : 0;
+  if (m <= 8) return dispatch_w8a8<false, false>(a, y_dtype, 1, st);
+  return y_dtype == LM_BF16 ? launch_w8a8<BF16, 16, false, false>(a, 1, st)
+                            : launch_w8a8<FP16, 16, false, false>(a, 1, st);
 }
 
 int w8a16_gemv_dense(const void *x, const int8_t *q, const float *s, void *y, int64_t m,

@@ -50,4 +50,10 @@ KsPlan ksplit_plan(int64_t m, int64_t n, int64_t k);
 int w8a16_ksplit(const KsPlan &plan, const void *x, const int8_t *q, const float *s, void *y,
                  int64_t m, int64_t n, int64_t k, int dtype, hipStream_t st);
 
+
+// W8A8 on few rows already quantized (gemv.hip): the same results as the GEMM.
+bool w8a8_gemv_serves(int64_t m, int64_t k);
+int w8a8_gemv_rows(const int8_t *xq, const float *xs, const int8_t *q, const float *s, void *y,
+                   int64_t m, int64_t n, int64_t k, int swiglu, int y_dtype, hipStream_t st);
+
 }  // namespace lm

@@ -12,15 +12,17 @@
 // library is compiled with -ffp-contract=off), so every fp32 accumulator, and
 // therefore its bf16 rounding, is bit-identical to the reference's.
 //
-// Tile: 128 rows x 128 columns per workgroup of four waves (2 x 2, 64 x 64
-// each); one K group (128 bytes of every A row and B row) per stage, staged in
-// LDS with a 16-byte row pad and prefetched into registers one group ahead.
+// Tile: 32 x 64 to 128 x 128 per workgroup of four waves (2 x 2); one K group
+// (128 bytes of every A row and B row) per stage, staged in LDS with a 16-byte
+// row pad and prefetched into registers one group ahead.
 // Within a 16x16x64 MFMA a lane holds row (lane & 15) and 16 consecutive K
 // bytes at offset 16 (lane >> 4) of the 64-K step, for A and B alike; the
 // order of K inside the sum does not matter because the int32 sum is exact.
 // The per-group epilogue (four fp32 operations per output element) costs
 // about as much issue time as the group's MFMAs, so the kernel's ceiling is
-// below the int8 MFMA peak by that ratio.
+// below the int8 MFMA peak by that ratio; its groups follow each other, so a
+// tile alone on its CU is a chain of K / 128 of them (8.5 us at K = 2048 for
+// the smallest tile, 25 for the largest).
 //
 // SwiGLU mode reads the n weight rows as [gate; up] halves: a tile's columns
 // pair gate column j with its up partner half + j in the same lane, and the
@@ -30,9 +32,6 @@
 namespace lm {
 namespace {
 
-constexpr int kQBM = 128;  // tile rows
-constexpr int kQBN = 128;  // tile columns
-constexpr int kQOcc = 2;   // workgroups per CU the register budget targets
 constexpr int kQG = 128;         // K group
 constexpr int kQPitch = kQG + 16;  // LDS bytes per staged row
 
@@ -47,31 +46,35 @@ struct W8A8GemmArgs {
   int64_t M;
   int N, K, ldy;
   int nt_count, mt_count;
+  bool cols_by_xcd;
 };
 
-template <typename T, bool SWIGLU, int BN, int OCC>
+// BM x BN tile, its four waves WM x (4 / WM).
+template <typename T, bool SWIGLU, int BM, int BN, int WM, int OCC>
 __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
-  constexpr int MI = 4, NI = BN / 32;  // 16x16 sub-tiles per wave (64 x BN/2)
-  constexpr int BCH = BN / 32;         // 16-byte B chunks per thread per group
-  __shared__ __align__(16) int8_t As[kQBM * kQPitch];
+  constexpr int WN = 4 / WM;
+  constexpr int MI = BM / WM / 16, NI = BN / WN / 16;  // 16x16 sub-tiles per wave
+  constexpr int ACH = BM / 32, BCH = BN / 32;  // 16-byte chunks per thread per group
+  static_assert(BM % 32 == 0 && BM + BN <= 256 && NI % 2 == 0, "tile shape");
+  __shared__ __align__(16) int8_t As[BM * kQPitch];
   __shared__ __align__(16) int8_t Bs[BN * kQPitch];
-  __shared__ float xsl[kQBM];
+  __shared__ float xsl[BM];
   __shared__ float wsl[BN];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  // All column tiles of one row tile run back to back on one XCD (linear id
-  // b is dealt to XCD b % 8), so the row tile's activations stay in its L2.
+  const int wm = wave / WN, wn = wave % WN;
+  // Linear id b runs on XCD b % 8: all row tiles of a column tile back to back
+  // on one XCD (cols_by_xcd), or all column tiles of a row tile.
   const int b = blockIdx.x;
   const int j = b >> 3;
-  const int mt = (j / a.nt_count) * 8 + (b & 7);
-  const int nt = j % a.nt_count;
-  if (mt >= a.mt_count) return;
+  const int mt = a.cols_by_xcd ? j % a.mt_count : (j / a.nt_count) * 8 + (b & 7);
+  const int nt = a.cols_by_xcd ? (j / a.mt_count) * 8 + (b & 7) : j % a.nt_count;
+  if (mt >= a.mt_count || nt >= a.nt_count) return;
 
-  const int64_t m0 = (int64_t)mt * kQBM;
-  const int rows = (int)min((int64_t)kQBM, a.M - m0);
+  const int64_t m0 = (int64_t)mt * BM;
+  const int rows = (int)min((int64_t)BM, a.M - m0);
   const int K = a.K;
   const int G = K / kQG;
   const int half = a.N >> 1;
@@ -89,9 +92,10 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
   };
   auto col_base = [&](int ni) -> int {
     if constexpr (SWIGLU) {
-      return ni < NI / 2 ? wn * (BN / 4) + ni * 16 : BN / 2 + wn * (BN / 4) + (ni - NI / 2) * 16;
+      return ni < NI / 2 ? wn * (8 * NI) + ni * 16
+                         : BN / 2 + wn * (8 * NI) + (ni - NI / 2) * 16;
     } else {
-      return wn * (BN / 2) + ni * 16;
+      return wn * (16 * NI) + ni * 16;
     }
   };
 
@@ -99,10 +103,10 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
   // 128-byte rows of the A and B tiles (row c / 8, chunk c % 8).  Rows past M
   // and columns past N re-read row 0 of the tile / weight row 0 and are never
   // stored.
-  const int8_t *asrc[4];
+  const int8_t *asrc[ACH];
   const int8_t *bsrc[BCH];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < ACH; ++i) {
     const int c = tid + 256 * i;
     const int r = c >> 3;
     asrc[i] = a.xq + (m0 + (r < rows ? r : 0)) * K + (c & 7) * 16;
@@ -113,22 +117,22 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
     const int wr = wrow(c >> 3);
     bsrc[i] = a.q + (int64_t)(wr >= 0 ? wr : 0) * K + (c & 7) * 16;
   }
-  // thread t < 128 carries the scale of tile row t, 128 <= t < 128 + BN that
-  // of column t - 128
+  // thread t < BM carries the scale of tile row t, BM <= t < BM + BN that of
+  // column t - BM
   const float *ssrc = nullptr;
-  if (tid < kQBM) {
+  if (tid < BM) {
     ssrc = a.xs + (m0 + (tid < rows ? tid : 0)) * G;
-  } else if (tid < kQBM + BN) {
-    const int wr = wrow(tid - kQBM);
+  } else if (tid < BM + BN) {
+    const int wr = wrow(tid - BM);
     ssrc = a.s + (int64_t)(wr >= 0 ? wr : 0) * G;
   }
 
-  u32x4 areg[4], breg[BCH];
+  u32x4 areg[ACH], breg[BCH];
   float sreg = 0.0f;
   auto prefetch = [&](int g) {
     const int k0 = g * kQG;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) areg[i] = ldg16(asrc[i] + k0);
+    for (int i = 0; i < ACH; ++i) areg[i] = ldg16(asrc[i] + k0);
 #pragma unroll
     for (int i = 0; i < BCH; ++i) breg[i] = ldg16(bsrc[i] + k0);
     if (ssrc) sreg = ssrc[g];
@@ -144,7 +148,7 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
   for (int g = 0; g < G; ++g) {
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < ACH; ++i) {
       const int c = tid + 256 * i;
       *reinterpret_cast<u32x4 *>(&As[(c >> 3) * kQPitch + (c & 7) * 16]) = areg[i];
     }
@@ -153,10 +157,10 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
       const int c = tid + 256 * i;
       *reinterpret_cast<u32x4 *>(&Bs[(c >> 3) * kQPitch + (c & 7) * 16]) = breg[i];
     }
-    if (tid < kQBM)
+    if (tid < BM)
       xsl[tid] = sreg;
-    else if (tid < kQBM + BN)
-      wsl[tid - kQBM] = sreg;
+    else if (tid < BM + BN)
+      wsl[tid - BM] = sreg;
     __syncthreads();
     if (g + 1 < G) prefetch(g + 1);
 
@@ -168,7 +172,7 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi)
         af[mi] = *reinterpret_cast<const i32x4 *>(
-            &As[(wm * 64 + mi * 16 + (lane & 15)) * kQPitch + kk]);
+            &As[(wm * 16 * MI + mi * 16 + (lane & 15)) * kQPitch + kk]);
 #pragma unroll
       for (int ni = 0; ni < NI; ++ni)
         bfr[ni] = *reinterpret_cast<const i32x4 *>(&Bs[(col_base(ni) + (lane & 15)) * kQPitch + kk]);
@@ -188,10 +192,11 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
     for (int mi = 0; mi < MI; ++mi) {
 #pragma unroll
       for (int it = 0; it < 4; ++it) {
-        const float xv = xsl[wm * 64 + mi * 16 + (lane >> 4) * 4 + it];
+        const float xv = xsl[wm * 16 * MI + mi * 16 + (lane >> 4) * 4 + it];
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni)
-          acc[mi][ni][it] = add_rn(acc[mi][ni][it], mul_rn(mul_rn((float)p[mi][ni][it], xv), wv[ni]));
+          acc[mi][ni][it] =
+              add_rn(acc[mi][ni][it], mul_rn(mul_rn((float)p[mi][ni][it], xv), wv[ni]));
       }
     }
   }
@@ -200,13 +205,13 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
   for (int mi = 0; mi < MI; ++mi) {
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
-      const int rl = wm * 64 + mi * 16 + (lane >> 4) * 4 + it;
+      const int rl = wm * 16 * MI + mi * 16 + (lane >> 4) * 4 + it;
       if (rl >= rows) continue;
       uint16_t *yrow = a.y + (m0 + rl) * a.ldy;
       if constexpr (SWIGLU) {
 #pragma unroll
         for (int ni = 0; ni < NI / 2; ++ni) {
-          const int col = n0 + wn * (BN / 4) + ni * 16 + (lane & 15);
+          const int col = n0 + wn * (8 * NI) + ni * 16 + (lane & 15);
           if (col < half) {
             const float gate = T::round(acc[mi][ni][it]);
             const float up = T::round(acc[mi][ni + NI / 2][it]);
@@ -222,6 +227,44 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
       }
     }
   }
+}
+
+template <typename T, int BM, int BN, int WM, int OCC>
+int launch_tile(W8A8GemmArgs a, bool swiglu, hipStream_t st) {
+  a.nt_count = (int)(swiglu ? cdiv(a.N / 2, BN / 2) : cdiv(a.N, BN));
+  a.mt_count = (int)cdiv(a.M, BM);
+  // Every XCD takes columns (a call of few rows would otherwise run on a few
+  // XCDs: [64, 2048] by [4096, 2048] 12.4 against 8.7 us) unless the row tiles
+  // come in eights and the rows are many ([2048, 2048] by [4096, 2048]: 36.3 us
+  // with a row tile's columns on one XCD, 38.1 without).
+  a.cols_by_xcd = a.N > 2 * a.M || a.mt_count % 8 != 0;
+  const int64_t grid = a.cols_by_xcd ? 8 * (int64_t)a.mt_count * ((a.nt_count + 7) / 8)
+                                     : 8 * (int64_t)a.nt_count * ((a.mt_count + 7) / 8);
+  LM_REQUIRE(grid < (int64_t(1) << 31), LM_EINVAL, "problem too large for one launch");
+  if (swiglu)
+    w8a8_mfma_kernel<T, true, BM, BN, WM, OCC><<<(unsigned)grid, 256, 0, st>>>(a);
+  else
+    w8a8_mfma_kernel<T, false, BM, BN, WM, OCC><<<(unsigned)grid, 256, 0, st>>>(a);
+  return check_launch("w8a8_mfma_kernel");
+}
+
+template <typename T>
+int launch_w8a8_tiles(const W8A8GemmArgs &a, bool swiglu, hipStream_t st) {
+  // The tile with the smallest estimated time at K = 2048 (all scale with K
+  // alike): a + b r us for r rounds of 256 tiles, measured from r = 1 to 16
+  // ([64, 2048] by [4096, 2048]: 8.7 us in 32 x 64 tiles, 25 in 128 x 128;
+  // [700, 2048] by [4096, 2048]: 19.5 us in 64 x 64, 26 in 128 x 128; [2048,
+  // 2048] by [4096, 2048]: 36 us in 128 x 128, 42 in 64 x 64).
+  const int64_t n = swiglu ? a.N / 2 : a.N;
+  auto rounds = [&](int bm, int bn) {
+    return (double)(((int64_t)cdiv(a.M, bm) * cdiv(n, swiglu ? bn / 2 : bn) + 255) / 256);
+  };
+  const double c0 = 5.5 + 3.1 * rounds(32, 64), c1 = 6.5 + 4.5 * rounds(64, 64),
+               c2 = 10.0 + 7.0 * rounds(64, 128), c3 = 15.0 + 11.0 * rounds(128, 128);
+  if (c0 <= c1 && c0 <= c2 && c0 <= c3) return launch_tile<T, 32, 64, 2, 4>(a, swiglu, st);
+  if (c1 <= c2 && c1 <= c3) return launch_tile<T, 64, 64, 2, 3>(a, swiglu, st);
+  if (c2 <= c3) return launch_tile<T, 64, 128, 2, 2>(a, swiglu, st);
+  return launch_tile<T, 128, 128, 2, 2>(a, swiglu, st);
 }
 
 }  // namespace
@@ -250,18 +293,8 @@ extern "C" int lm_w8a8_gemm(const int8_t *xq, const float *xs, const int8_t *q, 
   a.N = (int)n;
   a.K = (int)k;
   a.ldy = (int)(swiglu ? n / 2 : n);
-  a.nt_count = (int)(swiglu ? cdiv(n / 2, kQBN / 2) : cdiv(n, kQBN));
-  a.mt_count = (int)cdiv(m, kQBM);
-  const int64_t grid = 8 * (int64_t)a.nt_count * ((a.mt_count + 7) / 8);
-  LM_REQUIRE(grid < (int64_t(1) << 31), LM_EINVAL, "problem too large for one launch");
   hipStream_t st = as_stream(stream);
-  const bool bf = y_dtype == LM_BF16;
-  if (swiglu) {
-    if (bf) w8a8_mfma_kernel<BF16, true, kQBN, kQOcc><<<(unsigned)grid, 256, 0, st>>>(a);
-    else w8a8_mfma_kernel<FP16, true, kQBN, kQOcc><<<(unsigned)grid, 256, 0, st>>>(a);
-  } else {
-    if (bf) w8a8_mfma_kernel<BF16, false, kQBN, kQOcc><<<(unsigned)grid, 256, 0, st>>>(a);
-    else w8a8_mfma_kernel<FP16, false, kQBN, kQOcc><<<(unsigned)grid, 256, 0, st>>>(a);
-  }
-  return check_launch("w8a8_mfma_kernel");
+  if (w8a8_gemv_serves(m, k)) return w8a8_gemv_rows(xq, xs, q, s, y, m, n, k, swiglu, y_dtype, st);
+  return y_dtype == LM_BF16 ? launch_w8a8_tiles<BF16>(a, swiglu != 0, st)
+                            : launch_w8a8_tiles<FP16>(a, swiglu != 0, st);
 }

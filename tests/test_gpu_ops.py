@@ -117,6 +117,30 @@ def test_w8a8_gemm_bit_exact(dev, m, n, rows):
     assert torch.equal(w8a8.gemm(xq, xs, qd, sd), y)
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('m,n,k', [(1, 24, 2048), (9, 1000, 2048), (16, 34, 2048), (17, 1000, 2048),
+                                   (33, 130, 384), (700, 4096, 128), (1000, 1100, 256),
+                                   (1025, 4100, 128), (2100, 4000, 128)])
+def test_w8a8_gemm_tiles_bit_exact(dev, m, n, k, dtype):
+    """Every tile of the W8A8 GEMM (32 x 64 to 128 x 128, chosen by size) and
+    the K-parallel form of up to 16 rows, with ragged rows and columns: the
+    outputs of a sample of rows equal the oracle's bit for bit, SwiGLU within
+    the rounding of its exponential."""
+    rnd = O.bf16 if dtype == torch.bfloat16 else O.fp16
+    gen = seeded(m + n)
+    x = torch.randn(m, k, generator=gen).to(dtype)
+    wq, ws = O.quantize_weight((torch.randn(n, k, generator=gen) * 0.02).numpy())
+    qd, sd = torch.from_numpy(wq).to(dev), torch.from_numpy(ws).to(dev)
+    xq, xs = w8a8.quantize(x.to(dev))
+    sel = np.unique(np.r_[0, m - 1, np.random.default_rng(m).integers(0, m, 12)])
+    ref = O.w8a8_linear(x.float().numpy()[sel], wq, ws, rnd)
+    y = w8a8.gemm(xq, xs, qd, sd, out_dtype=dtype)
+    assert np.array_equal(y.float().cpu().numpy()[sel], ref)
+    h = w8a8.gemm(xq, xs, qd, sd, swiglu=True, out_dtype=dtype).float().cpu().numpy()[sel]
+    href = int8.swiglu(torch.from_numpy(ref).to(dtype).to(dev)).float().cpu().numpy()
+    assert np.array_equal(h, href)
+
+
 def _bank(gen, e, n, k, scale=0.02):
     w = torch.randn(e, n, k, generator=gen) * scale
     q, s = O.quantize_weight(w.numpy())
