@@ -84,6 +84,7 @@ class MoeLayer(ctypes.Structure):
 
 _lib = None
 _lock = threading.Lock()
+_fns = {}  # name -> bound function, filled when the library is loaded
 
 
 def lib():
@@ -100,6 +101,7 @@ def lib():
                     fn = getattr(handle, name)
                     fn.restype = res
                     fn.argtypes = args
+                    _fns[name] = fn
                 _lib = handle
     return _lib
 
@@ -117,22 +119,33 @@ def check(rc):
 
 
 def call(name, *args):
-    check(getattr(lib(), name)(*args))
+    if _lib is None:
+        lib()
+    rc = _fns[name](*args)
+    if rc:
+        check(rc)
 
 
 def ptr(t):
     return None if t is None else t.data_ptr()
 
 
+# A small call is bound by its host side, so the handle of the current stream
+# is read without building a Stream object (about 2 us) where torch offers it.
+_raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None)
+
+
 def stream(device=None):
+    if _raw_stream is not None and device is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
+_DTYPE_CODES = {torch.bfloat16: LM_BF16, torch.float16: LM_FP16, torch.float32: LM_FP32}
+
+
 def dtype_code(dtype):
-    if dtype == torch.bfloat16:
-        return LM_BF16
-    if dtype == torch.float16:
-        return LM_FP16
-    if dtype == torch.float32:
-        return LM_FP32
-    raise ValueError(f'unsupported dtype {dtype}')
+    code = _DTYPE_CODES.get(dtype)
+    if code is None:
+        raise ValueError(f'unsupported dtype {dtype}')
+    return code

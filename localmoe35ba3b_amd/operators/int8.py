@@ -9,6 +9,8 @@ has no counterpart: the whole expert bank is resident in HBM, so an
 Int8Experts module holds device tensors and builds its decode descriptor
 table on the device without a host synchronisation.
 """
+import functools
+
 import torch
 
 from .. import _lib
@@ -34,14 +36,15 @@ def linear(x, q, scale, large_tile=False):
     if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError('W8A16 requires CUDA FP16/BF16 activations')
     n, k = q.shape
-    if k % 128 or x.shape[-1] != k or tuple(scale.shape) != (n, k // 128):
+    shape = x.shape
+    if k % 128 or shape[-1] != k or scale.shape != (n, k // 128):
         raise ValueError('Invalid INT8 group geometry')
     _require_int8_pair(q, scale)
     x = x.contiguous()
-    m = x.numel() // k
-    out = torch.empty((*x.shape[:-1], n), device=x.device, dtype=x.dtype)
+    out = x.new_empty((*shape[:-1], n))
     _lib.call('lm_w8a16_linear', x.data_ptr(), q.data_ptr(), scale.data_ptr(), out.data_ptr(),
-              m, n, k, _lib.dtype_code(x.dtype), int(bool(large_tile)), _lib.stream(x.device))
+              x.numel() // k, n, k, _lib.dtype_code(x.dtype), 1 if large_tile else 0,
+              _lib.stream(x.device))
     return out
 
 
@@ -55,6 +58,9 @@ class Int8Linear(torch.nn.Module):
         self.large_prefill_tile = False
 
     def forward(self, x):
+        buffers = self._buffers  # skips two module attribute searches
+        if 'q' in buffers and 'scale' in buffers:
+            return linear(x, buffers['q'], buffers['scale'], self.large_prefill_tile)
         return linear(x, self.q, self.scale, self.large_prefill_tile)
 
 
@@ -102,11 +108,11 @@ def swiglu(gu):
 
 def _selection(ids):
     """The selected ids of one token as (flat contiguous tensor, element size)."""
-    if not ids.is_cuda or ids.dtype not in (torch.int64, torch.int32):
-        if not ids.is_cuda or ids.is_floating_point():
-            raise ValueError('Expected CUDA integer routing IDs')
+    if not ids.is_cuda or ids.is_floating_point():
+        raise ValueError('Expected CUDA integer routing IDs')
+    if ids.dtype is not torch.int64 and ids.dtype is not torch.int32:
         ids = ids.to(torch.int64)
-    return ids.reshape(-1).contiguous(), ids.element_size()
+    return ids.reshape(-1).contiguous(), 8 if ids.dtype is torch.int64 else 4
 
 
 def _bank_args(gate_up, down):
@@ -128,6 +134,11 @@ def build_descriptors(gate_up, down, ids):
     _lib.call('lm_expert_table', flat.data_ptr(), size, n, gate_up['q'].shape[0],
               *_bank_args(gate_up, down), table.data_ptr(), _lib.stream(flat.device))
     return table
+
+
+@functools.lru_cache(maxsize=None)
+def _decode_fits(n, hidden, intermediate):
+    return bool(_lib.lib().lm_w8a16_experts_decode_fits(n, hidden, intermediate))
 
 
 _w8a16_grouped_linear = grouped_linear  # the operator the two-launch decode computes
@@ -167,8 +178,7 @@ class Int8Experts(torch.nn.Module):
                                          self.large_tile)
         hidden, intermediate = x.shape[-1], self.down['q'].shape[-1]
         if (grouped_linear is _w8a16_grouped_linear
-                and _lib.lib().lm_w8a16_experts_decode_fits(top_k_index.numel(), hidden,
-                                                            intermediate)):
+                and _decode_fits(top_k_index.numel(), hidden, intermediate)):
             return self._decode(x, top_k_index, top_k_weights, hidden, intermediate)
         table = build_descriptors(self.gate_up, self.down, top_k_index)
         experts = table.shape[0]
@@ -185,8 +195,8 @@ class Int8Experts(torch.nn.Module):
         x, weights = x.contiguous(), weights.contiguous()
         flat, size = _selection(ids)
         n = flat.numel()
-        h = torch.empty((n, intermediate), dtype=x.dtype, device=x.device)
-        out = torch.empty((1, hidden), dtype=x.dtype, device=x.device)
+        h = x.new_empty((n, intermediate))
+        out = x.new_empty((1, hidden))
         _lib.call('lm_w8a16_experts_decode', x.data_ptr(), flat.data_ptr(), size, n,
                   self.gate_up['q'].shape[0], *_bank_args(self.gate_up, self.down),
                   weights.data_ptr(), _lib.dtype_code(weights.dtype), h.data_ptr(),

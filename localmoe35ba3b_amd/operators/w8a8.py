@@ -25,10 +25,11 @@ def quantize(x):
         raise ValueError('Expected CUDA rows with K divisible by 128')
     if x.dtype not in (torch.bfloat16, torch.float16):
         raise ValueError('Expected CUDA rows with K divisible by 128')
-    q = torch.empty_like(x, dtype=torch.int8)
-    s = torch.empty((x.shape[0], k // 128), device=x.device, dtype=torch.float32)
+    rows = x.shape[0]
+    q = x.new_empty((rows, k), dtype=torch.int8)
+    s = x.new_empty((rows, k // 128), dtype=torch.float32)
     _lib.call('lm_act_quant_g128', x.data_ptr(), _lib.dtype_code(x.dtype), q.data_ptr(),
-              s.data_ptr(), x.shape[0], k, _lib.stream(x.device))
+              s.data_ptr(), rows, k, _lib.stream(x.device))
     return q, s
 
 
@@ -69,14 +70,15 @@ def linear(x, q, scale, swiglu=False):
     x = x.contiguous()
     _check_rows(x)
     n, k = q.shape
-    if k % 128 or x.shape[-1] != k or tuple(scale.shape) != (n, k // 128):
+    m = x.shape[0]
+    if k % 128 or x.shape[-1] != k or scale.shape != (n, k // 128):
         raise ValueError('Invalid INT8 group geometry')
-    if x.shape[0] > 8:
+    if m > 8:
         xq, xs = quantize(x)
         return gemm(xq, xs, q, scale, swiglu, out_dtype=x.dtype)
-    out = torch.empty((x.shape[0], n // 2 if swiglu else n), device=x.device, dtype=x.dtype)
+    out = x.new_empty((m, n // 2 if swiglu else n))
     _lib.call('lm_w8a8_linear', x.data_ptr(), q.contiguous().data_ptr(),
-              scale.contiguous().data_ptr(), out.data_ptr(), x.shape[0], n, k, int(bool(swiglu)),
+              scale.contiguous().data_ptr(), out.data_ptr(), m, n, k, 1 if swiglu else 0,
               _lib.dtype_code(x.dtype), _lib.stream(x.device))
     return out
 
@@ -91,12 +93,12 @@ def gemm(xq, xs, q, scale, swiglu=False, out_dtype=torch.bfloat16):
         raise ValueError('Expected CUDA int8 rows and weights')
     m, k = xq.shape
     n = q.shape[0]
-    if (k % 128 or q.shape[1] != k or tuple(scale.shape) != (n, k // 128)
-            or tuple(xs.shape) != (m, k // 128)):
+    if (k % 128 or q.shape[1] != k or scale.shape != (n, k // 128)
+            or xs.shape != (m, k // 128)):
         raise ValueError('Invalid INT8 group geometry')
     if swiglu and n % 2:
         raise ValueError('SwiGLU needs an even number of weight rows')
-    out = torch.empty((m, n // 2 if swiglu else n), device=xq.device, dtype=out_dtype)
+    out = xq.new_empty((m, n // 2 if swiglu else n), dtype=out_dtype)
     _lib.call('lm_w8a8_gemm', xq.contiguous().data_ptr(), xs.contiguous().data_ptr(),
               q.contiguous().data_ptr(), scale.contiguous().data_ptr(), out.data_ptr(), m, n, k,
               int(bool(swiglu)), _lib.dtype_code(out_dtype), _lib.stream(xq.device))

@@ -25,9 +25,9 @@ def router_topk(hidden, weight, top_k, bias=None):
     if weight.shape[1] != h:
         raise ValueError('router weight does not match the hidden size')
     dev = hidden.device
-    logits = torch.empty((tokens, experts), dtype=torch.float32, device=dev)
-    ids = torch.empty((tokens, top_k), dtype=torch.int64, device=dev)
-    weights = torch.empty((tokens, top_k), dtype=torch.bfloat16, device=dev)
+    logits = hidden.new_empty((tokens, experts), dtype=torch.float32)
+    ids = hidden.new_empty((tokens, top_k), dtype=torch.int64)
+    weights = hidden.new_empty((tokens, top_k))
     if bias is not None:
         bias = bias.to(device=dev, dtype=torch.float32).contiguous()
     _lib.call('lm_router_topk', hidden.data_ptr(), weight.contiguous().data_ptr(), _lib.ptr(bias),

@@ -40,14 +40,13 @@ def plan(ids, experts, bm):
     tokens, top = ids.shape
     routes = tokens * top
     max_tiles = (routes + bm - 1) // bm + experts
-    dev = ids.device
-    pos = torch.empty(routes, dtype=torch.int64, device=dev)
-    table = torch.empty((max_tiles, 3), dtype=torch.int64, device=dev)
-    ordered = torch.empty((tokens, top), dtype=torch.int64, device=dev)
-    slots = torch.empty((tokens, top), dtype=torch.int64, device=dev)
+    pos = ids.new_empty(routes)
+    table = ids.new_empty((max_tiles, 3))
+    ordered = ids.new_empty((tokens, top))
+    slots = ids.new_empty((tokens, top))
     _lib.call('lm_route_plan', ids.data_ptr(), tokens, top, int(experts), int(bm), pos.data_ptr(),
               table.data_ptr(), max_tiles, ordered.data_ptr(), slots.data_ptr(),
-              _lib.stream(dev))
+              _lib.stream(ids.device))
     return pos, table, ordered, slots
 
 
@@ -55,9 +54,9 @@ def _check_bank(q, s):
     if q.dtype != torch.int8 or s.dtype != torch.float32 or q.ndim != 3 or s.ndim != 3:
         raise ValueError('Invalid INT8 group geometry')
     e, n, k = q.shape
-    if k % 128 or tuple(s.shape) != (e, n, k // 128):
+    if k % 128 or s.shape != (e, n, k // 128):
         raise ValueError('Invalid INT8 group geometry')
-    if q.stride(2) != 1 or q.stride(1) != k or s.stride(2) != 1 or s.stride(1) != k // 128:
+    if q.stride()[1:] != (k, 1) or s.stride()[1:] != (k // 128, 1):
         raise ValueError('Invalid INT8 group geometry')
 
 
@@ -86,7 +85,7 @@ def routed_gemm(x, q, s, pos, table, bm, gather):
 def routed_reduce(values, ordered, slots, weights, tokens, n):
     """Prefill combine (prefill._reduce): ascending-expert accumulation per
     token, rounded to the values' dtype at every step."""
-    out = torch.empty((tokens, n), device=values.device, dtype=values.dtype)
+    out = values.new_empty((tokens, n))
     weights = weights.contiguous()
     _lib.call('lm_routed_reduce', values.data_ptr(), ordered.data_ptr(), slots.data_ptr(),
               weights.data_ptr(), _lib.dtype_code(weights.dtype), out.data_ptr(), tokens, n,
@@ -104,11 +103,11 @@ def run_plan(x, weights, banks, pos, table, ordered, slots, bm, ready_event=None
         torch.cuda.current_stream().wait_event(ready_event)
     st = _lib.stream(x.device)
     code = _lib.dtype_code(x.dtype)
-    hidden = torch.empty((routes, qg.shape[1] // 2), device=x.device, dtype=x.dtype)
+    hidden = x.new_empty((routes, qg.shape[1] // 2))
     _lib.call('lm_routed_gate_up_swiglu', x.data_ptr(), x.shape[0], qg.data_ptr(), sg.data_ptr(),
               qg.shape[0], qg.stride(0), sg.stride(0), pos.data_ptr(), table.data_ptr(),
               table.shape[0], bm, hidden.data_ptr(), routes, qg.shape[1], qg.shape[2], code, st)
-    down = torch.empty((routes, qd.shape[1]), device=x.device, dtype=x.dtype)
+    down = x.new_empty((routes, qd.shape[1]))
     _lib.call('lm_routed_gemm_w8a16', hidden.data_ptr(), routes, qd.data_ptr(), sd.data_ptr(),
               qd.shape[0], qd.stride(0), sd.stride(0), pos.data_ptr(), table.data_ptr(),
               table.shape[0], bm, down.data_ptr(), routes, qd.shape[1], qd.shape[2], 0, code, st)
