@@ -278,6 +278,19 @@ int lm_router_topk(const void *x, const void *w, const float *bias,
                    int64_t experts, int64_t hidden, int64_t top_k,
                    void *stream);
 
+/* lm_router_topk with device scratch of the caller, for calls of many tokens,
+ * whose logits are then taken from exact int8 products (the same logits, ids
+ * and weights, faster).  lm_router_workspace_bytes says how much the call
+ * takes (0: the call uses none); workspace is 16-byte aligned, NULL runs
+ * lm_router_topk, a smaller one than stated is LM_ENOMEM.  Every byte read is
+ * written by the call first.  No counterpart in the reference (HF:768-776). */
+int64_t lm_router_workspace_bytes(int64_t tokens, int64_t experts, int64_t hidden);
+int lm_router_topk_ws(const void *x, const void *w, const float *bias,
+                      float *logits, int64_t *ids, void *weights,
+                      int64_t tokens, int64_t experts, int64_t hidden,
+                      int64_t top_k, void *workspace, int64_t workspace_bytes,
+                      void *stream);
+
 /* Qwen3_5MoeRMSNorm (HF:801-815): y = bf16(x * rsqrt(mean(x^2) + eps)
  * * (1 + w)); x, y bf16 [rows, n], w fp32 [n] (NULL = zeros). */
 int lm_rmsnorm(const void *x, const float *w, void *y, int64_t rows,

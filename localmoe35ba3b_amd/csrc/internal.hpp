@@ -6,6 +6,10 @@ namespace lm {
 
 int router_logits(const uint16_t *x, const uint16_t *w, const float *bias, float *logits,
                   int64_t T, int64_t E, int64_t H, hipStream_t st);
+// The same logits through int8 digits (router_digits.hip), which need a workspace.
+int64_t router_digits_bytes(int64_t T, int64_t E, int64_t H);
+int router_logits_digits(const uint16_t *x, const uint16_t *w, const float *bias, float *logits,
+                         int64_t T, int64_t E, int64_t H, void *workspace, hipStream_t st);
 int router_topk(const float *logits, int64_t T, int64_t E, int64_t K, int64_t *ids,
                 uint16_t *weights, hipStream_t st);
 int route_plan(const int64_t *ids, int64_t T, int64_t K, int64_t E, int64_t bm, int64_t *pos,

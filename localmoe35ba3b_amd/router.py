@@ -30,9 +30,11 @@ def router_topk(hidden, weight, top_k, bias=None):
     weights = hidden.new_empty((tokens, top_k))
     if bias is not None:
         bias = bias.to(device=dev, dtype=torch.float32).contiguous()
-    _lib.call('lm_router_topk', hidden.data_ptr(), weight.contiguous().data_ptr(), _lib.ptr(bias),
-              logits.data_ptr(), ids.data_ptr(), weights.data_ptr(), tokens, experts, h, top_k,
-              _lib.stream(dev))
+    need = _lib.lib().lm_router_workspace_bytes(tokens, experts, h)
+    workspace = hidden.new_empty(need, dtype=torch.uint8) if need else None
+    _lib.call('lm_router_topk_ws', hidden.data_ptr(), weight.contiguous().data_ptr(),
+              _lib.ptr(bias), logits.data_ptr(), ids.data_ptr(), weights.data_ptr(), tokens,
+              experts, h, top_k, _lib.ptr(workspace), need, _lib.stream(dev))
     return logits, weights, ids
 
 

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 import torch
 
-from localmoe35ba3b_amd import convert, router
+from localmoe35ba3b_amd import _lib, convert, router
 from localmoe35ba3b_amd.operators import int8, routing, w8a8
 from localmoe35ba3b_amd.runtime import gpu_routes, prefill
 from localmoe35ba3b_amd.runtime.stack import zipf_bias
@@ -400,6 +400,61 @@ def test_router_shapes(dev, t, e, h, k):
     assert np.array_equal(lg.cpu().numpy(), rl)
     assert np.array_equal(ids.cpu().numpy(), ri)
     assert np.abs(npf(wts) - rw).max() <= 2.0 ** -8
+
+
+def _direct_router(x, w, k, bias):
+    """router_topk without the workspace form (fp64 MFMA for every logit)."""
+    t, h = x.shape
+    e = w.shape[0]
+    lg = torch.empty(t, e, device=x.device)
+    ids = torch.empty(t, k, dtype=torch.int64, device=x.device)
+    wts = torch.empty(t, k, dtype=torch.bfloat16, device=x.device)
+    _lib.call('lm_router_topk', x.data_ptr(), w.data_ptr(), _lib.ptr(bias), lg.data_ptr(),
+              ids.data_ptr(), wts.data_ptr(), t, e, h, k, _lib.stream(x.device))
+    return lg, wts, ids
+
+
+@pytest.mark.parametrize('t,e,h,kind', [
+    (513, 256, 2048, 'normal'), (1000, 200, 768, 'normal'), (530, 17, 256, 'normal'),
+    (600, 256, 2048, 'outliers'), (520, 256, 1024, 'wide'), (515, 100, 4096, 'edges'),
+    (550, 256, 2048, 'ties')])
+def test_router_digits(dev, t, e, h, kind):
+    """The int8-digit form (more than 512 tokens) against the fp64 form, bit for
+    bit: ragged tiles, one to many K blocks, rows whose values leave the
+    23-bit grid ('outliers': a few channels 300 times the others; 'wide': values
+    from 2^-40 to 2^20, every logit open), rows of zeros, subnormals,
+    infinities and NaN ('edges'), and exact ties at bf16 rounding boundaries."""
+    assert _lib.lib().lm_router_workspace_bytes(t, e, h) > 0
+    g = torch.Generator(device=dev)
+    g.manual_seed(t)
+    x = torch.randn(t, h, generator=g, device=dev)
+    w = torch.randn(e, h, generator=g, device=dev) * 0.02
+    if kind == 'outliers':
+        x[:, ::301] *= 300
+    if kind == 'wide':
+        x = x * torch.exp2(torch.randint(-40, 21, (t, h), generator=g, device=dev).float())
+    if kind == 'edges':
+        x[3] = 0
+        x[5] *= 1e-38
+        x[6, 7] = float('inf')
+        x[8, 9] = float('nan')
+        x[10] *= 1e36
+        w[2] = 0
+        w[4] *= 1e-36
+        w[6, 1] = float('-inf')
+    if kind == 'ties':
+        x = torch.randint(-8, 9, (t, h), generator=g, device=dev).float()
+        w = torch.randint(-8, 9, (e, h), generator=g, device=dev).float()
+    x, w = x.to(torch.bfloat16), w.to(torch.bfloat16)
+    for bias in (None, torch.randn(e, generator=g, device=dev)):
+        got = router.router_topk(x, w, 4, bias)
+        ref = _direct_router(x, w, 4, bias)
+        assert torch.equal(got[0].view(torch.int32).where(~ref[0].isnan(), 0),
+                           ref[0].view(torch.int32).where(~ref[0].isnan(), 0))
+        assert torch.equal(got[0].isnan(), ref[0].isnan())
+        fine = ~ref[0].isnan().any(-1)
+        assert torch.equal(got[2][fine], ref[2][fine])
+        assert torch.equal(got[1][fine].view(torch.int16), ref[1][fine].view(torch.int16))
 
 
 def test_rmsnorm_bit_exact(dev):
