@@ -159,6 +159,12 @@ __global__ __launch_bounds__(kRdWaves * 64) void router_digits_kernel(DigitArgs 
 }
 
 constexpr int kRdTok = 32;  // tokens of a workgroup's tile
+// Above this many open logits of its 1024 a workgroup takes its whole tile by
+// fp64 MFMA instead of one dot product a wave and logit: with one value of each
+// row 30000 times the others, 2048 tokens took 140 us by dot products, 112 with
+// the line at 256, 76 at 128 (the direct form 45).  At 300 times the dot products
+// stay the cheaper way (39 us), and ordinary rows leave a handful.
+constexpr int kRdDense = 128;
 
 // A workgroup owns 32 tokens x 16 NJ experts, its waves the K blocks wave, wave
 // + 4, ...  The int32 sums of digit pairs of equal weight share an accumulator
@@ -276,6 +282,33 @@ __global__ __launch_bounds__(256, OCC) void router_digits_mfma(DigitArgs a) {
   }
   __syncthreads();
   const int n = n_open;
+  if (n > kRdDense) {  // uniform: every tile again, K in 32-wide stages as in route.hip
+    for (int own = 0; own < OWN; ++own) {
+      const int i = (4 * own + wave) / NJ, e = e0 + 16 * ((4 * own + wave) % NJ) + r;
+      const uint16_t *xr = a.x + (int64_t)min(t0 + 16 * i + r, a.T - 1) * a.H + 8 * q;
+      const uint16_t *wr = a.w + (int64_t)min(e, a.E - 1) * a.H + 8 * q;
+      f64x4 d[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+#pragma unroll 4
+      for (int k = 0; k < a.H; k += 32) {
+        const u32x4 xv = ldg16(xr + k), wv = ldg16(wr + k);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const uint32_t sh = (j & 1) ? 16u : 0u;
+          d[j & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+              (double)bf16_bits_to_f32((xv[j >> 1] >> sh) & 0xFFFFu),
+              (double)bf16_bits_to_f32((wv[j >> 1] >> sh) & 0xFFFFu), d[j & 1], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int t = t0 + 16 * i + 4 * it + q;  // fp64 tiles: row 4 it + q, column r
+        if (t >= a.T || e >= a.E) continue;
+        const float l = round_bf16((float)(d[0][it] + d[1][it]));
+        a.logits[(int64_t)t * a.E + e] = a.bias ? l + a.bias[e] : l;
+      }
+    }
+    return;
+  }
   for (int c = wave; c < n; c += 4) {
     const int t = t0 + open[c] / kRdExp, ee = e0 + open[c] % kRdExp;
     const uint16_t *xr = a.x + (int64_t)t * a.H, *wr = a.w + (int64_t)ee * a.H;
