@@ -4,7 +4,7 @@
 //   lm_w8a8_gemm for m <= 16 at K = 2048             (w8a8_gemv_rows)
 //   lm_w8a8_group_partials                           (exact int32 partials)
 //   lm_w8a16_grouped_gemv                            (int8.py:213-237)
-//   lm_w8a16_linear for m <= 8                       (int8.py:9-37)
+//   lm_w8a16_linear for few rows                     (int8.py:9-37)
 // All of them stream the weights with gemv_core.hpp; blockIdx.y selects the
 // expert of a descriptor table (grouped mode) or is 0 (dense mode).
 #include "gemv_core.hpp"

@@ -14,7 +14,7 @@
 //                          W8A8 (row-quantized SwiGLU output) / W8A16, then the
 //                          ascending-expert bf16 combine (int8.py:240-250), the
 //                          gated shared add and the residual add, in place.
-// Prefill runs: RMSNorm + shared gate, router (fp64 MFMA), top-k with
+// Prefill runs: RMSNorm + shared gate, approximate router (bf16 MFMA), exact top-k with
 // per-workgroup expert counts, the route plan scan (with the shared expert
 // appended as extra tiles), grouped W8A16 gate_up GEMM with fused SwiGLU,
 // grouped W8A16 down GEMM, and a per-token combine.

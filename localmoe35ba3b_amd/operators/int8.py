@@ -30,8 +30,8 @@ def linear(x, q, scale, large_tile=False):
     """y = x . bf16(q * s)^T with fp32 accumulation (int8.py:26-37).
 
     x: CUDA bf16/fp16 [..., K]; q int8 [N, K]; scale fp32 [N, K/128].
-    M <= 8 rows run the HBM-streaming GEMV, larger M the MFMA GEMM;
-    large_tile selects the taller MFMA tile like the reference flag.
+    One or two rows run the HBM-streaming GEMV, more the MFMA tiles their size
+    selects; large_tile selects the taller tile like the reference flag.
     """
     if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError('W8A16 requires CUDA FP16/BF16 activations')
@@ -108,8 +108,8 @@ def swiglu(gu):
 
 def _selection(ids):
     """The selected ids of one token as (flat contiguous tensor, element size)."""
-    if not ids.is_cuda or ids.is_floating_point():
-        raise ValueError('Expected CUDA integer routing IDs')
+    if not ids.is_cuda:
+        raise ValueError('Expected CUDA routing IDs')
     if ids.dtype is not torch.int64 and ids.dtype is not torch.int32:
         ids = ids.to(torch.int64)
     return ids.reshape(-1).contiguous(), 8 if ids.dtype is torch.int64 else 4
@@ -126,8 +126,15 @@ def build_descriptors(gate_up, down, ids):
 
     Returns a CUDA int64 [top_k, 5] table of (gate_up.q, gate_up.s, down.q,
     down.s) data pointers of each selected expert of the HBM bank plus its
-    slot, built by one kernel (no host read of the routing ids).
+    slot, built by one kernel (no host read of the routing ids).  Ids in host
+    memory give the same table there.
     """
+    if not ids.is_cuda:
+        experts, slots = torch.sort(ids.reshape(-1), stable=True)
+        experts = experts.to(torch.int64)
+        columns = [t.data_ptr() + experts * (t.stride(0) * t.element_size())
+                   for t in (gate_up['q'], gate_up['scale'], down['q'], down['scale'])]
+        return torch.stack([*columns, slots], dim=1)
     flat, size = _selection(ids)
     n = flat.numel()
     table = torch.empty((n, 5), dtype=torch.int64, device=flat.device)

@@ -65,8 +65,9 @@ def grouped_gemv(q, s, table, experts, n, field, shared, out_dtype=torch.bfloat1
 def linear(x, q, scale, swiglu=False):
     """Dense W8A8 linear of bf16 or fp16 rows: [M, N] or, with swiglu,
     [M, N/2], in x.dtype.  Up to 8 rows run as one fused quantize + GEMV
-    launch; more rows are quantized (quantize) and multiplied by the int8
-    MFMA GEMM (gemm)."""
+    launch; more rows are quantized (quantize) and multiplied by gemm: the
+    GEMV form while few rows keep it bound by the weights, int8 MFMA tiles
+    beyond."""
     x = x.contiguous()
     _check_rows(x)
     n, k = q.shape

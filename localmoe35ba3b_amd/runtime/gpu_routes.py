@@ -1,7 +1,7 @@
 """Device route plan and routed MoE (drop-in for qwen35_deploy/runtime/gpu_routes.py).
 
-plan        one-block HIP kernel: stable counting sort of the flat routing
-            ids, tile table, ordered/slots (gpu_routes.py:17-63) - no host
+plan        one HIP kernel: stable counting sort of the flat routing ids,
+            tile table, ordered/slots (gpu_routes.py:17-63) - no host
             synchronisation, no torch sort.
 routed_moe  plan -> grouped gate_up GEMM with the SwiGLU glue fused into the
             MFMA epilogue -> grouped down GEMM -> ordered combine

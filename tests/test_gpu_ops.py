@@ -278,13 +278,14 @@ def test_w8a16_grouped_and_experts_decode(dev):
 
 @pytest.mark.parametrize('n,hidden,inter,dtype,idt', [
     (8, 2048, 512, torch.bfloat16, torch.int64), (1, 2048, 512, torch.float16, torch.int64),
-    (3, 2048, 384, torch.bfloat16, torch.int32), (9, 2048, 512, torch.float16, torch.int64),
+    (3, 2048, 384, torch.bfloat16, torch.int32), (5, 2048, 512, torch.bfloat16, torch.float32), (9, 2048, 512, torch.float16, torch.int64),
     (12, 1024, 512, torch.bfloat16, torch.int64), (40, 384, 640, torch.bfloat16, torch.int64),
     (70, 256, 128, torch.bfloat16, torch.int64)])
 def test_experts_decode_forms(dev, n, hidden, inter, dtype, idt):
     """One token through Int8Experts against the separate operators, bit for
     bit: one to several batches of rows, widths other than the model's,
-    repeated ids, and more experts than the fused launches serve (70)."""
+    repeated ids, ids of other types, and more experts than the fused launches
+    serve (70)."""
     g = torch.Generator(device=dev)
     g.manual_seed(n + inter)
     e = 11
@@ -297,6 +298,7 @@ def test_experts_decode_forms(dev, n, hidden, inter, dtype, idt):
     x = torch.randn(1, hidden, generator=g, device=dev).to(dtype)
     out = int8.Int8Experts(0, gate_up, down)(x, ids, wts)
     table = int8.build_descriptors(gate_up, down, ids)
+    assert torch.equal(int8.build_descriptors(gate_up, down, ids.cpu()), table.cpu())
     order = torch.sort(ids.reshape(-1).long(), stable=True)
     assert torch.equal(table[:, 4], order.indices)
     for c, (t, size) in enumerate(((gq, 1), (gs, 4), (dq, 1), (ds, 4))):
