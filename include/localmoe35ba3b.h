@@ -95,6 +95,15 @@ int lm_w8a16_linear(const void *x, const int8_t *q, const float *s, void *y,
                     int64_t m, int64_t n, int64_t k, int dtype, int large_tile,
                     void *stream);
 
+/* What lm_w8a16_linear runs for a size (host only): form = {LM_LINEAR_*, tile
+ * rows, tile columns, 1 if a column tile's row tiles share an XCD (0: a row
+ * tile's columns do)}; tiles 0 for the GEMV. */
+#define LM_LINEAR_GEMV 0
+#define LM_LINEAR_KSPLIT 1   /* tiles whose waves split K */
+#define LM_LINEAR_STREAMED 2 /* weights streamed into registers */
+#define LM_LINEAR_LDS 3      /* weights staged in LDS */
+int lm_w8a16_linear_form(int64_t m, int64_t n, int64_t k, int64_t *form);
+
 /* Grouped W8A16 decode GEMV over a device descriptor table
  * table[e, 5] = {gate_up.q, gate_up.s, down.q, down.s, slot} (int64):
  * y[e, :] = x[shared ? 0 : e, :] . dequant(table[e, field..field+1])^T,
@@ -147,6 +156,10 @@ int lm_w8a8_linear(const void *x, const int8_t *q, const float *s, void *y,
 int lm_w8a8_gemm(const int8_t *xq, const float *xs, const int8_t *q, const float *s,
                  void *y, int64_t m, int64_t n, int64_t k, int swiglu, int y_dtype,
                  void *stream);
+
+/* What lm_w8a8_gemm runs for a size, as in lm_w8a16_linear_form
+ * (LM_LINEAR_GEMV or LM_LINEAR_LDS). */
+int lm_w8a8_gemm_form(int64_t m, int64_t n, int64_t k, int swiglu, int64_t *form);
 
 /* SwiGLU glue in `dtype` T: h[r, c] = T(T(silu(gu[r, c])) * gu[r, half + c]).
  * Replaces `gate, up = gu.chunk(2, -1); silu(gate) * up`

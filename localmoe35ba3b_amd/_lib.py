@@ -34,12 +34,14 @@ SIGNATURES = {
     'lm_w8_tile_rows': (I32, [P, I64, I64, I64, I64, P, I32, P]),
     'lm_act_quant_g128': (I32, [P, I32, P, P, I64, I64, P]),
     'lm_w8a16_linear': (I32, [P, P, P, P, I64, I64, I64, I32, I32, P]),
+    'lm_w8a16_linear_form': (I32, [I64, I64, I64, P]),
     'lm_w8a16_grouped_gemv': (I32, [P, P, P, I64, I64, I64, I32, I32, I32, P]),
     'lm_w8a8_grouped_gemv': (I32, [P, P, P, P, I64, I64, I64, I32, I32, I32, P]),
     'lm_w8a8_grouped_linear': (I32, [P, P, P, I64, I64, I64, I32, I32, I32, P]),
     'lm_w8a8_group_partials': (I32, [P, P, P, I64, I64, I64, P]),
     'lm_w8a8_linear': (I32, [P, P, P, P, I64, I64, I64, I32, I32, P]),
     'lm_w8a8_gemm': (I32, [P, P, P, P, P, I64, I64, I64, I32, I32, P]),
+    'lm_w8a8_gemm_form': (I32, [I64, I64, I64, I32, P]),
     'lm_swiglu': (I32, [P, P, I64, I64, I32, P]),
     'lm_ordered_reduce': (I32, [P, P, P, I32, P, I64, I64, I32, P]),
     'lm_expert_table': (I32, [P, I32, I64, I64, P, P, P, P, I64, I64, I64, I64, P, P]),

@@ -109,6 +109,21 @@ __device__ __forceinline__ void dequant16(u32x4 w, float s, uint32_t out[8]) {
   }
 }
 
+// Workgroups are dealt to the 8 XCDs round-robin by linear id.  Maps linear id
+// b to a (row tile, column tile): all column tiles of one row tile on one XCD,
+// back to back, so that its activation rows are fetched once and served from
+// that XCD's L2; with by_columns all row tiles of one column tile, which shares
+// its weights.  Launch xcd_grid (internal.hpp) workgroups; false for padding
+// ones.  One division serves both forms.
+__device__ __forceinline__ bool xcd_tile(int row_tiles, int col_tiles, bool by_columns, int &mt,
+                                         int &nt) {
+  const uint32_t b = blockIdx.x, j = b >> 3, inner = by_columns ? row_tiles : col_tiles;
+  const int outer = (int)(j / inner * 8 + (b & 7)), in = (int)(j % inner);
+  mt = by_columns ? in : outer;
+  nt = by_columns ? outer : in;
+  return outer < (by_columns ? col_tiles : row_tiles);
+}
+
 // Eight int8 weights -> eight T(q * s): the signed byte converts exactly
 // (v_cvt_f32_i32 with a sign-extended byte operand), so q * s is the
 // correctly rounded fp32 product, then RNE to T - bit-identical to

@@ -23,6 +23,7 @@
 // Dense calls of fewer rows run the K-split tiles of ksplit.hip.
 // In SwiGLU mode a tile's columns pair every gate column with its up partner
 // in the same lane.
+#include <algorithm>
 #include <type_traits>
 
 #include "internal.hpp"
@@ -59,34 +60,9 @@ struct GemmArgs {
   int nt_count;   // column tiles
   int mt_count;   // row tiles (table rows, or dense M tiles)
   bool few_rows;     // routed: few rows per expert on average (kFewRows)
-  bool cols_by_xcd;  // dense: a column tile's row tiles share an XCD, not a row tile's columns
+  bool wide;         // dense: 256-column tiles
+  bool by_columns;   // dense: how the tiles are dealt to the XCDs (xcd_tile)
 };
-
-// Workgroups are dealt to the 8 XCDs round-robin by linear id.  Map linear
-// id b -> (row tile, column tile) so that all column tiles of one row tile
-// run on the same XCD back to back: the gathered activation rows of a tile
-// are then read from HBM/MALL once and served from that XCD's L2 for the
-// other column tiles.  With cols_by_xcd (dense) the roles are swapped.
-// Returns false for padding workgroups.
-__device__ __forceinline__ bool xcd_tile(const GemmArgs &a, int &mt, int &nt) {
-  const int b = blockIdx.x;
-  const int j = b >> 3;
-  if (a.cols_by_xcd) {
-    mt = j % a.mt_count;
-    nt = (j / a.mt_count) * 8 + (b & 7);
-    return nt < a.nt_count;
-  }
-  mt = (j / a.nt_count) * 8 + (b & 7);
-  nt = j % a.nt_count;
-  return mt < a.mt_count;
-}
-
-// Workgroups of an XCD-mapped launch; callers reject counts beyond one
-// launch's grid (2^31 - 1) before launching.
-static int64_t xcd_grid(int64_t mtiles, int64_t ntiles, bool cols_by_xcd = false) {
-  if (cols_by_xcd) return 8 * mtiles * ((ntiles + 7) / 8);
-  return 8 * ntiles * ((mtiles + 7) / 8);
-}
 
 template <typename T, int BM, int WM, bool SWIGLU, bool GATHER, bool DENSE>
 __global__ __launch_bounds__(256) void w8a16_mfma_kernel(GemmArgs a) {
@@ -105,7 +81,7 @@ __global__ __launch_bounds__(256) void w8a16_mfma_kernel(GemmArgs a) {
   const int wm = wave / WN;
   const int wn = wave % WN;
   int mt, nt;
-  if (!xcd_tile(a, mt, nt)) return;
+  if (!xcd_tile(a.mt_count, a.nt_count, a.by_columns, mt, nt)) return;
 
   int64_t e = 0, start;
   int rows;
@@ -292,7 +268,7 @@ __global__ __launch_bounds__(256) void grouped_mfma_kernel(GemmArgs a) {
   const int lane = tid & 63;
   const int wn = tid >> 6;
   int mt, nt;
-  if (!xcd_tile(a, mt, nt)) return;
+  if (!xcd_tile(a.mt_count, a.nt_count, a.by_columns, mt, nt)) return;
   const TileBounds tb = tile_bounds(a.table[mt * 3], a.table[mt * 3 + 1], a.table[mt * 3 + 2],
                                     a.experts, a.y_rows, a.tile_rows);
   if (tb.rows <= 0) return;
@@ -854,7 +830,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void grouped_rb_kernel(GemmArgs a) {
   constexpr int SC_BYTES = NW * TN * (K / 128) * 4 + (WL == kWlTilesF16 ? (NW * TN + BM) * 4 : 0);
   __shared__ __align__(16) unsigned char smem[3 * BM * 128 * HL + SC_BYTES];
   int mt, nt;
-  if (!xcd_tile(a, mt, nt)) return;
+  if (!xcd_tile(a.mt_count, a.nt_count, a.by_columns, mt, nt)) return;
   // Gathered rows on the tile copies: this tile's rows of the tile-major
   // gather map, requested before the table row and independently of it
   // (the rows rb_tile assigns to this lane for the tallest tile, and to
@@ -970,7 +946,7 @@ static int launch_rb(GemmArgs a, unsigned mtiles, hipStream_t st) {
   constexpr int RBN = NW * TN;
   a.nt_count = SWIGLU ? (int)cdiv(a.N / 2, RBN / 2) : (int)cdiv(a.N, RBN);
   a.mt_count = (int)mtiles;
-  const int64_t grid = xcd_grid(a.mt_count, a.nt_count, a.cols_by_xcd);
+  const int64_t grid = xcd_grid(a.mt_count, a.nt_count, a.by_columns);
   LM_REQUIRE(grid < (int64_t(1) << 31), LM_EINVAL, "problem too large for one launch");
   grouped_rb_kernel<T, SWIGLU, GATHER, WL, K, BM, TN, kRbBD, kRbHL, AD, NW, OCC,
                     DEEP><<<(unsigned)grid, NW * 64, 0, st>>>(a);
@@ -984,12 +960,11 @@ static int launch_grouped(GemmArgs a, unsigned mtiles, hipStream_t st) {
   if (mtiles == 0) return LM_OK;
   if constexpr (WL == kWlDirect && !SWIGLU && !GATHER) {
     if (!a.table) {  // dense rows, K = 512, 2048 or 4096
-      const bool wide = (int64_t)mtiles * cdiv(a.N, kRbNWWide * kRbTN) >= kRbWideTiles;
       auto go = [&](auto k_tag) -> int {
         constexpr int KC = decltype(k_tag)::value;
         if (a.tile_rows != kRbBMTall) return launch_rb<T, false, false, WL, KC>(a, mtiles, st);
-        return wide ? launch_rb<T, false, false, WL, KC, kRbBMTall, kRbNWWide>(a, mtiles, st)
-                    : launch_rb<T, false, false, WL, KC, kRbBMTall>(a, mtiles, st);
+        return a.wide ? launch_rb<T, false, false, WL, KC, kRbBMTall, kRbNWWide>(a, mtiles, st)
+                      : launch_rb<T, false, false, WL, KC, kRbBMTall>(a, mtiles, st);
       };
       if (a.K == 4096) return go(std::integral_constant<int, 4096>{});
       if (a.K == 2048) return go(std::integral_constant<int, 2048>{});
@@ -1024,8 +999,87 @@ static int launch_gemm(GemmArgs a, unsigned mtiles, hipStream_t st) {
   return check_launch("w8a16_mfma_kernel");
 }
 
-int w8a16_gemm_dense(const void *x, const int8_t *q, const float *s, void *y, int64_t m,
-                     int64_t n, int64_t k, int dtype, int large_tile, hipStream_t st) {
+// The XCD deal of a dense matrix: the fewer rounds of tiles on the busiest XCD.
+// A column tile's rows on one XCD leave XCDs without work where there are fewer
+// than 8 column tiles ([20000, 2048] by [64, 2048]: 87 us against 26 the other
+// way), a row tile's columns on one XCD where there are few row tiles or one
+// beyond a multiple of 8 ([1300, 2048] by [3000, 2048]: 37 against 27).  Beside
+// the rounds count the load within them, at a twentieth ([2100, 4096] by [4096,
+// 4096] of W8A8 tiles: 68 tiles 86 us, 96 in as many rounds 92), and what an XCD
+// reads: n + m / 4 or n / 8 + 2 m times K bytes with 2-byte activations, and 5700
+// of n - 2 m weigh as a round ([780, 2048] by [8192, 2048]: 42 us by columns in 3
+// rounds, 51 by rows in 2.1).  Over 260 sizes of register-streamed tiles, 470 of
+// K-split tiles and 560 of W8A8 tiles this is 0.4 % slower than the better of both.
+XcdDeal xcd_deal(int64_t m, int64_t n, int64_t row_tiles, int64_t col_tiles, int tile_rows,
+                 bool short_tail, int act_bytes) {
+  auto rounds = [](int64_t tiles) { return (double)((tiles + 31) / 32); };
+  const int64_t col_load = row_tiles * ((col_tiles + 7) / 8);
+  const int64_t tail = m % tile_rows, full = row_tiles - (tail ? 1 : 0);
+  const int64_t full_load = col_tiles * ((full + 7) / 8);
+  double by_rows = rounds(full_load), row_load = (double)full_load;
+  if (tail) {
+    // the XCD of the last row tile: its columns follow those of full / 8 others
+    const int64_t before = col_tiles * (full / 8);
+    const int64_t extra = col_tiles - ((int64_t)rounds(before) * 32 - before);
+    const double part = short_tail ? (double)tail / tile_rows : 1.0;
+    by_rows = std::max(by_rows, rounds(before) + part * rounds(std::max<int64_t>(extra, 0)));
+    row_load = std::max(row_load, (double)before + part * (double)col_tiles);
+  }
+  const double by_cols = rounds(col_load);
+  const bool by_columns = by_cols + 0.05 * (double)col_load / 32.0 <
+                          by_rows + 0.05 * row_load / 32.0 + (double)(n - act_bytes * m) / 5700.0;
+  return XcdDeal{by_columns, by_columns ? by_cols : by_rows};
+}
+
+// What a dense call of m rows runs.
+struct DenseForm {
+  int kernel;  // LM_LINEAR_*
+  KsPlan ks;   // of LM_LINEAR_KSPLIT
+  int rows, cols;  // of a tile
+  bool by_columns;
+};
+
+static DenseForm dense_form(int64_t m, int64_t n, int64_t k) {
+  const KsPlan ks = ksplit_plan(m, n, k);
+  DenseForm f{LM_LINEAR_KSPLIT, ks, ks.rows, ks.cols, ks.by_columns};
+  if (m <= 8) {
+    // One or two rows stream the weights through the GEMV (lm_head
+    // [248320, 2048]: 77 against 92 us on K-split tiles); from three rows on
+    // the GEMV's dot products cost more than the weights (200 against 93 us;
+    // at N = 4096 and 8 rows 6.9 against 4.1 us), and at K = 512 one round of
+    // K-split tiles is the shorter chain (2.6 against 3.4 us).
+    if (ks.shape >= 0 && (m > 2 || (k == 512 && n <= 256 * 16))) return f;
+    return DenseForm{LM_LINEAR_GEMV, ks, 0, 0, false};
+  }
+  // Other K: the LDS-dequant kernel.
+  if (ks.shape < 0) return DenseForm{LM_LINEAR_LDS, ks, 128, kBN, false};
+  // K = 512, 2048 or 4096: small tiles whose waves split K (ksplit.hip) or the
+  // register-streamed kernel over 96-row tiles (128-row tiles from
+  // kDenseTallM rows; no tile table), whichever is estimated to be faster.  A
+  // register-streamed tile walks K alone, and a round of them takes that long
+  // however many run; further rounds overlap with the one before.  Fitted
+  // in us at K = 512, 2048 and 4096: one round of 96 x 128 tiles 8.8, 20.5 and
+  // 36 to 42, two 12.3, 30 and 58; of 128 x 128 10.2, 24.5 and 43.5, two 14.5, 36
+  // and 67; of 128 x 256 15.7, 39 and 70, two 25.6, 67 and 125.  The K-split tiles
+  // take 5 to 20 us while one or two rounds of them hold the matrix (x [45, 2048]
+  // by [4096, 2048]: 6.9 us; [333, 4096] by [2048, 4096]: 17 against 41), and
+  // lose where the rows fill the tall tiles ([700, 2048] by [4096, 2048]: 32
+  // against 22 us).
+  const double kk = (double)k / 2048.0;
+  const int bm = m >= kDenseTallM ? kRbBMTall : 96;
+  const int64_t mt = cdiv(m, bm);
+  const bool wide = bm == kRbBMTall && mt * cdiv(n, kRbNWWide * kRbTN) >= kRbWideTiles;
+  const int bn = (wide ? kRbNWWide : kRbNW) * kRbTN;
+  const XcdDeal deal = xcd_deal(m, n, mt, cdiv(n, bn), bm, true, 2);
+  const double cost = wide              ? 6.0 + 1.5 * kk + (2.0 + 30.0 * kk) * deal.rounds
+                      : bm == kRbBMTall ? 4.2 + 8.0 * kk + (1.5 + 11.0 * kk) * deal.rounds
+                                        : 3.3 + 7.7 * kk + (0.9 + 9.3 * kk) * deal.rounds;
+  if (ks.cost <= cost) return f;
+  return DenseForm{LM_LINEAR_STREAMED, ks, bm, bn, deal.by_columns};
+}
+
+static int w8a16_gemm_dense(const DenseForm &f, const void *x, const int8_t *q, const float *s,
+                            void *y, int64_t m, int64_t n, int64_t k, int dtype, hipStream_t st) {
   GemmArgs a{};
   a.x = static_cast<const uint16_t *>(x);
   a.ldx = k;
@@ -1036,35 +1090,13 @@ int w8a16_gemm_dense(const void *x, const int8_t *q, const float *s, void *y, in
   a.ldy = n;
   a.N = (int)n;
   a.K = (int)k;
-  (void)large_tile;
-  // K = 512, 2048 or 4096: small tiles whose waves split K (ksplit.hip) or the
-  // register-streamed kernel over 96-row tiles (128-row tiles from
-  // kDenseTallM rows; no tile table), whichever is estimated to be faster.  A
-  // 96 x 128 tile walks K alone and takes about 21.5 us at K = 2048 (8.5 us
-  // with its launch at 512, 41 us at 4096) whether one or 256 of them run;
-  // each further round of 256 tiles adds about half of that.  The K-split tiles take 4 to
-  // 20 us while one or two rounds of them hold the matrix (x [45, 2048] by
-  // [4096, 2048]: 6.9 against 20.5 us; [333, 4096] by [2048, 4096]: 17
-  // against 41), and lose where the rows fill the tall tiles ([700, 2048] by
-  // [4096, 2048]: 30 against 24 us).  Other K keeps the LDS-dequant kernel.
-  const KsPlan plan = ksplit_plan(m, n, k);
-  if (plan.shape >= 0) {
-    const int bm = m >= kDenseTallM ? kRbBMTall : 96;
-    const int64_t rounds = ((int64_t)cdiv(m, bm) * cdiv(n, kRbNW * kRbTN) + 255) / 256;
-    const double rb_cost = (2.0 + 19.5 * (double)k / 2048.0) * (0.55 + 0.45 * (double)rounds);
-    if (plan.cost <= rb_cost) return w8a16_ksplit(plan, x, q, s, y, m, n, k, dtype, st);
-    a.tile_rows = bm;
-    // All row tiles of a column tile on one XCD: every XCD has work whatever
-    // the number of row tiles, and reads only its part of the weights
-    // ([100, 2048] by [8192, 2048]: 22.8 us against 31.3 with a row tile's
-    // columns on one XCD; [2048, 2048] by [8192, 2048]: 76 against 82).  Whole
-    // rounds of row tiles with at least as many bytes as the weights keep
-    // their columns together ([2048, 2048] by [4096, 2048]: 38.9 against 39.2).
-    a.cols_by_xcd = n > 2 * m || cdiv(m, bm) % 8 != 0;
-    return dtype == LM_BF16 ? launch_grouped<BF16, false, false, kWlDirect>(a, cdiv(m, bm), st)
-                            : launch_grouped<FP16, false, false, kWlDirect>(a, cdiv(m, bm), st);
-  }
-  const unsigned mt = cdiv(m, 128);
+  a.tile_rows = f.rows;
+  a.wide = f.cols == kRbNWWide * kRbTN;
+  a.by_columns = f.by_columns;
+  const unsigned mt = cdiv(m, f.rows);
+  if (f.kernel == LM_LINEAR_STREAMED)
+    return dtype == LM_BF16 ? launch_grouped<BF16, false, false, kWlDirect>(a, mt, st)
+                            : launch_grouped<FP16, false, false, kWlDirect>(a, mt, st);
   if (dtype == LM_BF16) return launch_gemm<BF16, 128, 2, false, false, true>(a, mt, st);
   return launch_gemm<FP16, 128, 2, false, false, true>(a, mt, st);
 }
@@ -1143,19 +1175,22 @@ extern "C" int lm_w8a16_linear(const void *x, const int8_t *q, const float *s, v
              "Invalid INT8 group geometry");
   if (m == 0) return LM_OK;
   LM_REQUIRE(x && q && s && y, LM_EINVAL, "null pointer");
-  if (m <= 8) {
-    // One or two rows stream the weights through the GEMV (lm_head
-    // [248320, 2048]: 77 against 92 us on K-split tiles); from three rows on
-    // the GEMV's dot products cost more than the weights (200 against 93 us;
-    // at N = 4096 and 8 rows 6.9 against 4.1 us), and at K = 512 one round of
-    // K-split tiles is the shorter chain (2.6 against 3.4 us).
-    const KsPlan plan = ksplit_plan(m, n, k);
-    if (plan.shape >= 0 && (m > 2 || (k == 512 && n <= 256 * 16)))
-      return w8a16_ksplit(plan, x, q, s, y, m, n, k, dtype, as_stream(stream));
-    return w8a16_gemv_dense(x, q, s, y, m, n, k, dtype, as_stream(stream));
-  }
+  (void)large_tile;
   LM_REQUIRE(m < (1LL << 31), LM_EINVAL, "Invalid INT8 group geometry");
-  return w8a16_gemm_dense(x, q, s, y, m, n, k, dtype, large_tile, as_stream(stream));
+  hipStream_t st = as_stream(stream);
+  const DenseForm f = dense_form(m, n, k);
+  if (f.kernel == LM_LINEAR_GEMV) return w8a16_gemv_dense(x, q, s, y, m, n, k, dtype, st);
+  if (f.kernel == LM_LINEAR_KSPLIT) return w8a16_ksplit(f.ks, x, q, s, y, m, n, k, dtype, st);
+  return w8a16_gemm_dense(f, x, q, s, y, m, n, k, dtype, st);
+}
+
+extern "C" int lm_w8a16_linear_form(int64_t m, int64_t n, int64_t k, int64_t *form) {
+  LM_REQUIRE(k > 0 && k % 128 == 0 && n > 0 && n < (1LL << 31) && m > 0 && m < (1LL << 31) && form,
+             LM_EINVAL, "Invalid INT8 group geometry");
+  const DenseForm f = dense_form(m, n, k);
+  const int64_t v[4] = {f.kernel, f.rows, f.cols, f.by_columns};
+  std::copy(v, v + 4, form);
+  return LM_OK;
 }
 
 static int check_routed(const RoutedGemm &r) {

@@ -43,17 +43,34 @@ struct RoutedGemm {
 };
 int routed_gemm(const RoutedGemm &r, hipStream_t st);
 
+// How a dense matrix of row_tiles x col_tiles tiles is dealt to the 8 XCDs of 32
+// CUs (xcd_tile, common.hpp), and the rounds of one tile per CU that the busiest
+// XCD works through.  short_tail: the last row tile takes time by its rows;
+// act_bytes: of an activation, 0 where an XCD's L2 holds them all.
+struct XcdDeal {
+  bool by_columns;
+  double rounds;
+};
+XcdDeal xcd_deal(int64_t m, int64_t n, int64_t row_tiles, int64_t col_tiles, int tile_rows,
+                 bool short_tail, int act_bytes);
+// Workgroups of such a launch; callers reject counts beyond one launch's grid
+// (2^31 - 1) before launching.
+inline int64_t xcd_grid(int64_t row_tiles, int64_t col_tiles, bool by_columns = false) {
+  return by_columns ? 8 * row_tiles * ((col_tiles + 7) / 8) : 8 * col_tiles * ((row_tiles + 7) / 8);
+}
+
 // Dense W8A16 over small tiles whose waves split K (ksplit.hip): the tile
 // shape for an [m, n, k] problem (shape < 0: k not served) with its estimated
 // time in us, and the launch.
 struct KsPlan {
   int shape;
   double cost;
+  int rows, cols;  // of a tile
+  bool by_columns;
 };
 KsPlan ksplit_plan(int64_t m, int64_t n, int64_t k);
 int w8a16_ksplit(const KsPlan &plan, const void *x, const int8_t *q, const float *s, void *y,
                  int64_t m, int64_t n, int64_t k, int dtype, hipStream_t st);
-
 
 // W8A8 on few rows already quantized (gemv.hip): the same results as the GEMM.
 bool w8a8_gemv_serves(int64_t m, int64_t k);

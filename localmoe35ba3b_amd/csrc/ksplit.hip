@@ -44,6 +44,7 @@ struct KsArgs {
   int64_t M;
   int N, K;
   int nt_count, mt_count;
+  bool by_columns;
 };
 
 // NU: units per wave (K / 64 / kKsWaves).  D: units held in registers, D - 1 of
@@ -63,13 +64,8 @@ __global__ __launch_bounds__(kKsWaves * 64) void ksplit_kernel(KsArgs a) {
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int p = lane >> 4, r = lane & 15;
-  // All row tiles of one column tile on one XCD (linear id b runs on XCD
-  // b % 8): its weights are fetched once and served from that XCD's L2.
-  const int b = blockIdx.x;
-  const int i = b >> 3;
-  const int mt = i % a.mt_count;
-  const int nt = (i / a.mt_count) * 8 + (b & 7);
-  if (nt >= a.nt_count) return;
+  int mt, nt;
+  if (!xcd_tile(a.mt_count, a.nt_count, a.by_columns, mt, nt)) return;
   const int64_t m0 = (int64_t)mt * (16 * MS);
   const int n0 = nt * BN;
   const int K = a.K;
@@ -190,7 +186,7 @@ int launch_ks(KsArgs a, hipStream_t st) {
   constexpr int D = D0 < NU ? D0 : NU;
   a.mt_count = (int)cdiv(a.M, 16 * MS);
   a.nt_count = (int)cdiv(a.N, 16 * NI);
-  const int64_t grid = 8 * (int64_t)a.mt_count * cdiv(a.nt_count, 8);
+  const int64_t grid = xcd_grid(a.mt_count, a.nt_count, a.by_columns);
   LM_REQUIRE(grid < (int64_t(1) << 31), LM_EINVAL, "problem too large for one launch");
   ksplit_kernel<T, MS, NI, NU, D><<<(unsigned)grid, kKsWaves * 64, 0, st>>>(a);
   return check_launch("ksplit_kernel");
@@ -218,22 +214,28 @@ int launch_k(const KsArgs &a, int shape, hipStream_t st) {
 
 }  // namespace
 
-// The tile shape with the smallest estimated time (in us beside the launch),
-// for a chip of 256 CUs that works through the tiles in whole rounds.  One
-// round takes about 0.8 us per 16 rows or columns and 2048 of K (loads,
-// staging, dequantization) plus 0.15 us per 16 x 16 tile (the sum over the
-// waves): measured at K = 512, 2048 and 4096 from 2.6 us (1 x 1, K = 512) to
-// 17 us (4 x 4, K = 4096).  Activations beyond an XCD's 4 MB L2 cost a quarter more.
+// The tile shape with the smallest estimated time in us, for 8 XCDs of 32 CUs
+// that work through their tiles in whole rounds.  A call takes 1.8 us, and a
+// round 0.8 us per 16 rows or columns and 2048 of K (loads, staging,
+// dequantization) plus 0.18 us per 16 x 16 tile (the sum over the waves):
+// measured at K = 512, 2048 and 4096 from 4.7 us (1 x 1, one round) to 36 us (4
+// x 4 at K = 4096, two rounds; 10 of 800 sizes further than 20 % off).  A tile's
+// rows are all loaded, so a short last row tile counts whole.  Where the
+// activations fit an XCD's 4 MB L2, every XCD may read all of them ([512, 2048]
+// by [512, 2048]: 6.5 us by columns, 7.0 by rows in one round both); beyond it
+// that costs a tenth.
 KsPlan ksplit_plan(int64_t m, int64_t n, int64_t k) {
-  KsPlan best{-1, 0.0};
+  KsPlan best{-1, 0.0, 0, 0, false};
   if (k != 512 && k != 2048 && k != 4096) return best;
+  const bool in_l2 = 2 * m * k <= (4 << 20);
   for (int i = 0; i < kKsCount; ++i) {
     const int ms = kKsShapes[i][0], ni = kKsShapes[i][1];
-    const int64_t tiles = (int64_t)cdiv(m, 16 * ms) * cdiv(n, 16 * ni);
-    const double cost = (double)((tiles + 255) / 256) *
-                        (0.15 * ms * ni + 0.8 * (ms + ni) * (double)k / 2048.0) *
-                        (2 * m * k > (4 << 20) ? 1.25 : 1.0);
-    if (best.shape < 0 || cost < best.cost) best = KsPlan{i, cost};
+    const int64_t mt = cdiv(m, 16 * ms), nt = cdiv(n, 16 * ni);
+    const XcdDeal deal = xcd_deal(m, n, mt, nt, 16 * ms, false, in_l2 ? 0 : 2);
+    const double round = 0.18 * ms * ni + 0.8 * (ms + ni) * (double)k / 2048.0;
+    const double cost = 1.8 + deal.rounds * round * (deal.by_columns && !in_l2 ? 1.1 : 1.0);
+    if (best.shape < 0 || cost < best.cost)
+      best = KsPlan{i, cost, 16 * ms, 16 * ni, deal.by_columns};
   }
   return best;
 }
@@ -248,6 +250,7 @@ int w8a16_ksplit(const KsPlan &plan, const void *x, const int8_t *q, const float
   a.M = m;
   a.N = (int)n;
   a.K = (int)k;
+  a.by_columns = plan.by_columns;
   return dtype == LM_BF16 ? launch_k<BF16>(a, plan.shape, st) : launch_k<FP16>(a, plan.shape, st);
 }
 

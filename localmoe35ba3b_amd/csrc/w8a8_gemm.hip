@@ -46,7 +46,7 @@ struct W8A8GemmArgs {
   int64_t M;
   int N, K, ldy;
   int nt_count, mt_count;
-  bool cols_by_xcd;
+  bool by_columns;
 };
 
 // BM x BN tile, its four waves WM x (4 / WM).
@@ -65,13 +65,8 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
-  // Linear id b runs on XCD b % 8: all row tiles of a column tile back to back
-  // on one XCD (cols_by_xcd), or all column tiles of a row tile.
-  const int b = blockIdx.x;
-  const int j = b >> 3;
-  const int mt = a.cols_by_xcd ? j % a.mt_count : (j / a.nt_count) * 8 + (b & 7);
-  const int nt = a.cols_by_xcd ? (j / a.mt_count) * 8 + (b & 7) : j % a.nt_count;
-  if (mt >= a.mt_count || nt >= a.nt_count) return;
+  int mt, nt;
+  if (!xcd_tile(a.mt_count, a.nt_count, a.by_columns, mt, nt)) return;
 
   const int64_t m0 = (int64_t)mt * BM;
   const int rows = (int)min((int64_t)BM, a.M - m0);
@@ -229,17 +224,42 @@ __global__ __launch_bounds__(256, OCC) void w8a8_mfma_kernel(W8A8GemmArgs a) {
   }
 }
 
+struct W8A8Form {
+  int rows, cols;  // of a tile
+  int64_t row_tiles, col_tiles;
+  bool by_columns;
+};
+
+// The tile with the smallest estimated time at K = 2048 (all scale with K
+// alike): a + b r us for r rounds of a tile per CU, measured from r = 1 to 16
+// ([64, 2048] by [4096, 2048]: 8.7 us in 32 x 64 tiles, 25 in 128 x 128; [700,
+// 2048] by [4096, 2048]: 19.5 us in 64 x 64, 26 in 128 x 128; [2048, 2048] by
+// [4096, 2048]: 36 us in 128 x 128, 42 in 64 x 64).  In SwiGLU mode a tile's
+// columns are pairs of weight rows.
+W8A8Form w8a8_form(int64_t m, int64_t n, bool swiglu) {
+  constexpr int tiles[4][2] = {{32, 64}, {64, 64}, {64, 128}, {128, 128}};
+  constexpr double first[4] = {5.5, 6.5, 10.0, 15.0}, each[4] = {3.1, 4.5, 7.0, 11.0};
+  W8A8Form best{};
+  double best_cost = 0.0;
+  for (int i = 0; i < 4; ++i) {
+    const int bm = tiles[i][0], bn = tiles[i][1];
+    const int64_t mt = cdiv(m, bm), nt = swiglu ? cdiv(n / 2, bn / 2) : cdiv(n, bn);
+    const XcdDeal deal = xcd_deal(m, n, mt, nt, bm, false, 1);
+    const double cost = first[i] + each[i] * deal.rounds;
+    if (!best.rows || cost < best_cost) {
+      best = W8A8Form{bm, bn, mt, nt, deal.by_columns};
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 template <typename T, int BM, int BN, int WM, int OCC>
-int launch_tile(W8A8GemmArgs a, bool swiglu, hipStream_t st) {
-  a.nt_count = (int)(swiglu ? cdiv(a.N / 2, BN / 2) : cdiv(a.N, BN));
-  a.mt_count = (int)cdiv(a.M, BM);
-  // Every XCD takes columns (a call of few rows would otherwise run on a few
-  // XCDs: [64, 2048] by [4096, 2048] 12.4 against 8.7 us) unless the row tiles
-  // come in eights and the rows are many ([2048, 2048] by [4096, 2048]: 36.3 us
-  // with a row tile's columns on one XCD, 38.1 without).
-  a.cols_by_xcd = a.N > 2 * a.M || a.mt_count % 8 != 0;
-  const int64_t grid = a.cols_by_xcd ? 8 * (int64_t)a.mt_count * ((a.nt_count + 7) / 8)
-                                     : 8 * (int64_t)a.nt_count * ((a.mt_count + 7) / 8);
+int launch_tile(W8A8GemmArgs a, const W8A8Form &f, bool swiglu, hipStream_t st) {
+  a.nt_count = (int)f.col_tiles;
+  a.mt_count = (int)f.row_tiles;
+  a.by_columns = f.by_columns;
+  const int64_t grid = xcd_grid(f.row_tiles, f.col_tiles, f.by_columns);
   LM_REQUIRE(grid < (int64_t(1) << 31), LM_EINVAL, "problem too large for one launch");
   if (swiglu)
     w8a8_mfma_kernel<T, true, BM, BN, WM, OCC><<<(unsigned)grid, 256, 0, st>>>(a);
@@ -250,21 +270,11 @@ int launch_tile(W8A8GemmArgs a, bool swiglu, hipStream_t st) {
 
 template <typename T>
 int launch_w8a8_tiles(const W8A8GemmArgs &a, bool swiglu, hipStream_t st) {
-  // The tile with the smallest estimated time at K = 2048 (all scale with K
-  // alike): a + b r us for r rounds of 256 tiles, measured from r = 1 to 16
-  // ([64, 2048] by [4096, 2048]: 8.7 us in 32 x 64 tiles, 25 in 128 x 128;
-  // [700, 2048] by [4096, 2048]: 19.5 us in 64 x 64, 26 in 128 x 128; [2048,
-  // 2048] by [4096, 2048]: 36 us in 128 x 128, 42 in 64 x 64).
-  const int64_t n = swiglu ? a.N / 2 : a.N;
-  auto rounds = [&](int bm, int bn) {
-    return (double)(((int64_t)cdiv(a.M, bm) * cdiv(n, swiglu ? bn / 2 : bn) + 255) / 256);
-  };
-  const double c0 = 5.5 + 3.1 * rounds(32, 64), c1 = 6.5 + 4.5 * rounds(64, 64),
-               c2 = 10.0 + 7.0 * rounds(64, 128), c3 = 15.0 + 11.0 * rounds(128, 128);
-  if (c0 <= c1 && c0 <= c2 && c0 <= c3) return launch_tile<T, 32, 64, 2, 4>(a, swiglu, st);
-  if (c1 <= c2 && c1 <= c3) return launch_tile<T, 64, 64, 2, 3>(a, swiglu, st);
-  if (c2 <= c3) return launch_tile<T, 64, 128, 2, 2>(a, swiglu, st);
-  return launch_tile<T, 128, 128, 2, 2>(a, swiglu, st);
+  const W8A8Form f = w8a8_form(a.M, a.N, swiglu);
+  if (f.rows == 32) return launch_tile<T, 32, 64, 2, 4>(a, f, swiglu, st);
+  if (f.rows == 128) return launch_tile<T, 128, 128, 2, 2>(a, f, swiglu, st);
+  if (f.cols == 64) return launch_tile<T, 64, 64, 2, 3>(a, f, swiglu, st);
+  return launch_tile<T, 64, 128, 2, 2>(a, f, swiglu, st);
 }
 
 }  // namespace
@@ -297,4 +307,18 @@ extern "C" int lm_w8a8_gemm(const int8_t *xq, const float *xs, const int8_t *q, 
   if (w8a8_gemv_serves(m, k)) return w8a8_gemv_rows(xq, xs, q, s, y, m, n, k, swiglu, y_dtype, st);
   return y_dtype == LM_BF16 ? launch_w8a8_tiles<BF16>(a, swiglu != 0, st)
                             : launch_w8a8_tiles<FP16>(a, swiglu != 0, st);
+}
+
+extern "C" int lm_w8a8_gemm_form(int64_t m, int64_t n, int64_t k, int swiglu, int64_t *form) {
+  LM_REQUIRE(m > 0 && m <= (int64_t(1) << 31) / 128, LM_EINVAL, "invalid row count");
+  LM_REQUIRE(n > 0 && n <= (1 << 24) && k > 0 && k % 128 == 0 && k <= 65536 && form, LM_EINVAL,
+             "Invalid INT8 group geometry");
+  LM_REQUIRE(!swiglu || n % 2 == 0, LM_EINVAL, "SwiGLU needs an even number of rows");
+  const bool gemv = w8a8_gemv_serves(m, k);
+  const W8A8Form f = gemv ? W8A8Form{} : w8a8_form(m, n, swiglu != 0);
+  form[0] = gemv ? LM_LINEAR_GEMV : LM_LINEAR_LDS;
+  form[1] = f.rows;
+  form[2] = f.cols;
+  form[3] = f.by_columns;
+  return LM_OK;
 }

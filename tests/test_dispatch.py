@@ -1,0 +1,55 @@
+"""CPU checks of the rules that choose a kernel and tile for a size, through
+the host queries of the C ABI.  No kernel is launched here."""
+import ctypes
+
+import pytest
+
+from localmoe35ba3b_amd import _lib
+
+GEMV, KSPLIT, STREAMED, LDS = range(4)
+SIZES = [(m, n) for n in (16, 64, 128, 256, 512, 1000, 2048, 4096, 8192)
+         for m in (9, 45, 130, 333, 700, 1023, 1024, 1100, 1900, 2048, 3000, 4096, 10000, 20000)]
+
+
+def linear_form(m, n, k):
+    form = (ctypes.c_int64 * 4)()
+    assert _lib.lib().lm_w8a16_linear_form(m, n, k, form) == _lib.LM_OK
+    return tuple(form)
+
+
+def w8a8_form(m, n, k, swiglu=False):
+    form = (ctypes.c_int64 * 4)()
+    assert _lib.lib().lm_w8a8_gemm_form(m, n, k, int(swiglu), form) == _lib.LM_OK
+    return tuple(form)
+
+
+def _rounds(m, n, rows, cols):
+    """Rounds of the busiest of 8 XCDs of 32 CUs, one tile a CU: with a row
+    tile's columns on one XCD, and with a column tile's rows."""
+    rt, ct = -(-m // rows), -(-n // cols)
+    return [-(-tiles // 32) for tiles in (ct * -(-rt // 8), rt * -(-ct // 8))]
+
+
+@pytest.mark.parametrize('kind', ['w8a16 512', 'w8a16 2048', 'w8a16 4096', 'w8a8 2048'])
+def test_tiles_are_dealt_to_all_xcds(kind):
+    """No XCD works through rounds of tiles that the other way to deal them
+    would have spread: the chosen way takes at most one round more (a short
+    last row tile, or less to read for each XCD), and no more than the other
+    where the matrix has few columns."""
+    name, k = kind.split()
+    for m, n in SIZES:
+        kernel, rows, cols, by_columns = (linear_form if name == 'w8a16' else w8a8_form)(
+            m, n, int(k))
+        if kernel == GEMV:
+            continue
+        taken, other = _rounds(m, n, rows, cols)[::-1 if by_columns else 1]
+        assert taken <= other + (1 if n > 2 * m or (m % rows and not by_columns) else 0), (m, n)
+        assert n > 1000 or taken <= max(other, 1), (m, n)
+
+
+def test_short_last_row_tile_stays_with_its_columns():
+    """[1060, 2048] by [4096, 2048] ends in a row tile of 36 rows: with whole
+    row tiles on an XCD the nine take little longer than eight (29 us), dealt
+    by columns two rounds (36)."""
+    assert linear_form(1060, 4096, 2048) == (STREAMED, 128, 128, 0)
+    assert linear_form(1280, 4096, 2048) == (STREAMED, 128, 128, 1)
