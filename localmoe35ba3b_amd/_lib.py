@@ -134,6 +134,13 @@ def ptr(t):
     return None if t is None else t.data_ptr()
 
 
+def device_table(table, experts):
+    """A descriptor table that kernels follow: `experts` rows of 5 int64 on the GPU."""
+    if not table.is_cuda or table.dtype is not torch.int64 or table.numel() < 5 * experts:
+        raise ValueError('Expected a CUDA int64 [experts, 5] descriptor table')
+    return table.contiguous()
+
+
 # A small call is bound by its host side, so the handle of the current stream
 # is read without building a Stream object (about 2 us) where torch offers it.
 _raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None)

@@ -64,6 +64,12 @@ class Int8Linear(torch.nn.Module):
         return linear(x, self.q, self.scale, self.large_prefill_tile)
 
 
+def _check_weights(weights, experts):
+    if not weights.is_cuda or weights.numel() < experts:
+        raise ValueError('Expected CUDA routing weights of every selected expert')
+    return weights.contiguous()
+
+
 def grouped_linear(x, table, experts, n, field, shared):
     """W8A16 grouped decode GEMV over a device descriptor table (int8.py:233-237).
 
@@ -72,7 +78,7 @@ def grouped_linear(x, table, experts, n, field, shared):
     """
     if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError('W8A16 requires CUDA FP16/BF16 activations')
-    x = x.contiguous()
+    x, table = x.contiguous(), _lib.device_table(table, experts)
     out = torch.empty((experts, n), dtype=x.dtype, device=x.device)
     _lib.call('lm_w8a16_grouped_gemv', x.data_ptr(), table.data_ptr(), out.data_ptr(),
               experts, n, x.shape[-1], field, int(bool(shared)), _lib.dtype_code(x.dtype),
@@ -87,9 +93,9 @@ def ordered_reduce(values, table, weights, out=None):
     weights [1, top_k] (bf16, fp16 or fp32); returns [1, N] in T.
     """
     experts, n = values.shape
+    table, weights = _lib.device_table(table, experts), _check_weights(weights, experts)
     if out is None:
         out = torch.empty((1, n), dtype=values.dtype, device=values.device)
-    weights = weights.contiguous()
     _lib.call('lm_ordered_reduce', values.contiguous().data_ptr(), table.data_ptr(),
               weights.data_ptr(), _lib.dtype_code(weights.dtype), out.data_ptr(), n, experts,
               _lib.dtype_code(values.dtype), _lib.stream(values.device))
@@ -124,10 +130,10 @@ def _bank_args(gate_up, down):
 def build_descriptors(gate_up, down, ids):
     """Decode descriptor table for one token, sorted by expert id (int8.py:164-179).
 
-    Returns a CUDA int64 [top_k, 5] table of (gate_up.q, gate_up.s, down.q,
+    Returns an int64 [top_k, 5] table of (gate_up.q, gate_up.s, down.q,
     down.s) data pointers of each selected expert of the HBM bank plus its
     slot, built by one kernel (no host read of the routing ids).  Ids in host
-    memory give the same table there.
+    memory give the same table there; the operators take it only on the GPU.
     """
     if not ids.is_cuda:
         experts, slots = torch.sort(ids.reshape(-1), stable=True)
@@ -199,9 +205,9 @@ class Int8Experts(torch.nn.Module):
         with the results of the separate operators."""
         if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16):
             raise ValueError('W8A16 requires CUDA FP16/BF16 activations')
-        x, weights = x.contiguous(), weights.contiguous()
         flat, size = _selection(ids)
         n = flat.numel()
+        x, weights = x.contiguous(), _check_weights(weights, n)
         h = x.new_empty((n, intermediate))
         out = x.new_empty((1, hidden))
         _lib.call('lm_w8a16_experts_decode', x.data_ptr(), flat.data_ptr(), size, n,

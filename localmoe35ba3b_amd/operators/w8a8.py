@@ -45,6 +45,7 @@ def grouped_linear(x, table, experts, n, field, shared):
     kernel.  x bf16 or fp16; the output is in x.dtype (w8a8.py:46)."""
     x = x.contiguous()
     _check_rows(x)
+    table = _lib.device_table(table, experts)
     out = torch.empty((experts, n), device=x.device, dtype=x.dtype)
     _lib.call('lm_w8a8_grouped_linear', x.data_ptr(), table.data_ptr(), out.data_ptr(), experts,
               n, x.shape[-1], field, int(bool(shared)), _lib.dtype_code(x.dtype),
@@ -55,6 +56,7 @@ def grouped_linear(x, table, experts, n, field, shared):
 def grouped_gemv(q, s, table, experts, n, field, shared, out_dtype=torch.bfloat16):
     """Grouped W8A8 GEMV on pre-quantized activations (the _linear kernel,
     w8a8.py:25-41); the output in out_dtype (bf16 or fp16)."""
+    table = _lib.device_table(table, experts)
     out = torch.empty((experts, n), device=q.device, dtype=out_dtype)
     _lib.call('lm_w8a8_grouped_gemv', q.contiguous().data_ptr(), s.contiguous().data_ptr(),
               table.data_ptr(), out.data_ptr(), experts, n, q.shape[-1], field, int(bool(shared)),
