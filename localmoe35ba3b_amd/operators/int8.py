@@ -154,7 +154,8 @@ def _decode_fits(n, hidden, intermediate):
     return bool(_lib.lib().lm_w8a16_experts_decode_fits(n, hidden, intermediate))
 
 
-_w8a16_grouped_linear = grouped_linear  # the operator the two-launch decode computes
+# The operators that the two-launch decode computes.
+_w8a16_decode = (build_descriptors, grouped_linear, swiglu, ordered_reduce)
 
 
 class Int8Experts(torch.nn.Module):
@@ -168,8 +169,9 @@ class Int8Experts(torch.nn.Module):
         device-planned routed MoE (gpu_routes.routed_moe);
       * M == 1: grouped decode - module-level grouped_linear (W8A16, or W8A8
         after `int8.grouped_linear = w8a8.grouped_linear`), SwiGLU, and the
-        ordered bf16 combine in ascending expert order; while grouped_linear
-        is the W8A16 operator, in two fused launches with the same results.
+        ordered bf16 combine in ascending expert order; while none of these
+        module-level operators is replaced, in two fused launches with the
+        same results.
     """
 
     def __init__(self, layer, gate_up, down, cache=None):
@@ -190,7 +192,7 @@ class Int8Experts(torch.nn.Module):
             return gpu_routes.routed_moe(x, top_k_weights, top_k_index.contiguous(), banks,
                                          self.large_tile)
         hidden, intermediate = x.shape[-1], self.down['q'].shape[-1]
-        if (grouped_linear is _w8a16_grouped_linear
+        if ((build_descriptors, grouped_linear, swiglu, ordered_reduce) == _w8a16_decode
                 and _decode_fits(top_k_index.numel(), hidden, intermediate)):
             return self._decode(x, top_k_index, top_k_weights, hidden, intermediate)
         table = build_descriptors(self.gate_up, self.down, top_k_index)

@@ -1,5 +1,5 @@
-"""CPU checks that operators refuse host memory that a kernel would follow.
-Tensors that only claim to be on the GPU reach the checks; nothing is launched."""
+"""CPU checks of the operator layer: host memory that a kernel would follow is
+refused, and replaced module-level operators are called.  Tensors that only claim to be on the GPU reach the checks; nothing is launched."""
 import pytest
 import torch
 
@@ -65,3 +65,21 @@ def test_experts_refuse_host_routing(launches, monkeypatch, swap):
         assert launches == []
         experts(gpu(X), gpu(ids), gpu(weights))
         assert launches == ['lm_w8a16_experts_decode']
+
+
+@pytest.mark.parametrize('name', ['build_descriptors', 'grouped_linear', 'swiglu',
+                                  'ordered_reduce'])
+def test_experts_call_replaced_operators(launches, monkeypatch, name):
+    """One decode token runs a program's own operator where it replaced one at
+    module level, and the fused launches where it did not."""
+    empty = torch.empty
+    monkeypatch.setattr(torch, 'empty', lambda *a, device=None, **kw: gpu(empty(*a, **kw)))
+    experts, ids = _experts(), gpu(torch.zeros(1, 4, dtype=torch.int64))
+    experts(gpu(X), ids, gpu(torch.zeros(1, 4)))
+    assert launches == ['lm_w8a16_experts_decode']
+    calls, original = [], getattr(int8, name)
+    monkeypatch.setattr(int8, name, lambda *a, **kw: calls.append(name) or original(*a, **kw))
+    experts(gpu(X), ids, gpu(torch.zeros(1, 4)))
+    assert calls == [name] * (2 if name == 'grouped_linear' else 1)
+    assert launches[1:] == ['lm_expert_table', 'lm_w8a16_grouped_gemv', 'lm_swiglu',
+                            'lm_w8a16_grouped_gemv', 'lm_ordered_reduce']
