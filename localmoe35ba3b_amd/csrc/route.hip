@@ -189,13 +189,12 @@ int router_logits(const uint16_t *x, const uint16_t *w, const float *bias, float
 }
 
 // Calls of more than kDigitTokens tokens take the int8 digits where the caller
-// brings a workspace for them (with the top-k, 21 us against 27 at 513 tokens,
-// 32 against 45 at 2048, 46 against 83 at 4096; up to 512 tokens the fp64 tiles
-// run in one round, 17 us).  Beyond 65536 tokens the digits would take over
-// 400 MB.
+// brings a workspace for them (with the top-k, 21 us against 26 at 513 tokens,
+// 31 against 45 at 2048, 46 against 83 at 4096; up to 512 tokens the fp64 tiles
+// run in one round, 17 us).
 constexpr int64_t kDigitTokens = 512;
 static bool router_digits_serves(int64_t T, int64_t H) {
-  return T > kDigitTokens && T <= 65536 && H % 256 == 0 && H <= 4096;
+  return T > kDigitTokens && H % 256 == 0 && H <= 4096;
 }
 
 int router_topk(const float *logits, int64_t T, int64_t E, int64_t K, int64_t *ids,

@@ -16,11 +16,21 @@
 // and every logit of a row that is not finite or below 2^-100, are taken again
 // by an fp64 dot product, the value the direct form computes.
 //
-// At that size router_digits_kernel takes 13.7 us (it writes 14 MB of digits;
+// Rows with a strong channel (some 200 times the others and more) would leave many
+// logits open, so a block of 16 token rows with a residue above kRdResidue
+// also stores its residues: x[k] - X[k] 2^-s has at most 8 significant bits and is
+// exact in bf16, and one bf16 product per logit adds sum_k (x - X 2^-s) w in
+// fp32, which leaves 2^-11 of the bound above.  With a channel of 3000 or 30000
+// times the others, 2048 tokens take 45 us (the direct form 46); without the
+// residues they took 77 and 76.
+//
+// At 2048 tokens router_digits_kernel takes 13.7 us (it writes 14 MB of digits;
 // half of that is its chain of load, largest value, barrier, digits) and
 // router_digits_mfma 15 us (4 us of MFMAs; its operands come from L2 at 200 MB
 // a call, and the 64-bit finish is not overlapped): 32 us with the top-k against
 // 45; 22 against 27 at 700 tokens, 46 against 83 at 4096.
+#include <algorithm>
+
 #include "internal.hpp"
 
 namespace lm {
@@ -41,8 +51,19 @@ struct DigitArgs {
   float *logits;
   int8_t *xd, *wd;
   RowMeta *xm, *wm;
+  u32x4 *xr;    // token residues x - X 2^-s, scaled by 2^s, bf16 in MFMA operand order:
+                // K block b of row block j holds two steps of 64 pieces at ((j nk + b) 2 + h) 64
+  uint8_t *xflag;  // [row blocks][halves of K]: the residues are stored
   int T, E, H;
 };
+
+// A half row block stores its residues where its 16 rows have more than
+// kRdResidue in all, in units of each row's grid and counting up to one per wave (a
+// sixteenth of the half row), so that one row alone does not decide.  A half row of
+// normal values has 0.03, with a channel 300 times the others 2 (11 logits of a
+// tile's 1024 open, taken again in 6 us of a call), 1000 times 7 (34 open, 17 us;
+// the residues 13).
+constexpr int kRdResidue = 80;
 
 // One 16-row block per workgroup, K blocks dealt to its 16 waves: coalesced row
 // loads into LDS (chunks XOR-swizzled by row), then lane l (row l & 15, quarter p
@@ -55,9 +76,10 @@ __global__ __launch_bounds__(kRdWaves * 64) void router_digits_kernel(DigitArgs 
   extern __shared__ __align__(16) unsigned char smem[];  // [16][H] values
   __shared__ uint32_t wmax[kRdWaves][16];
   __shared__ float wres[kRdWaves][16];
+  __shared__ int large;  // the block's residues in sixteenths of a grid unit
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tblocks = (a.T + 15) / 16;
+  const int tblocks = (a.T + 15) / 16;  // the expert rows' blocks follow
   const bool tok = (int)blockIdx.x < tblocks;
   const int blk = tok ? blockIdx.x : blockIdx.x - tblocks;
   const int rows = min(16, (tok ? a.T : a.E) - blk * 16);
@@ -88,6 +110,10 @@ __global__ __launch_bounds__(kRdWaves * 64) void router_digits_kernel(DigitArgs 
     const int ch = 8 * kb + 2 * p + h;
     return *reinterpret_cast<const u32x4 *>(smem + r * pitch + ((ch ^ (r & 7)) * 16));
   };
+  // scaled value j of a piece, and its distance from the grid
+  auto scaled = [](u32x4 v, int j, int s) {
+    return ldexpf(bf16_bits_to_f32((v[j >> 1] >> (16 * (j & 1))) & 0xFFFFu), s);
+  };
   uint32_t mb = 0;  // largest |x| as bits: the order of finite values, inf and NaN above
   for (int kb = wave; kb < nk; kb += kRdWaves)
 #pragma unroll
@@ -100,6 +126,7 @@ __global__ __launch_bounds__(kRdWaves * 64) void router_digits_kernel(DigitArgs 
   mb = max(mb, (uint32_t)__shfl_xor((int)mb, 16, 64));
   mb = max(mb, (uint32_t)__shfl_xor((int)mb, 32, 64));
   if (p == 0) wmax[wave][r] = mb;
+  if (threadIdx.x == 0) large = 0;
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < kRdWaves; ++w) mb = max(mb, wmax[w][r]);
@@ -118,7 +145,7 @@ __global__ __launch_bounds__(kRdWaves * 64) void router_digits_kernel(DigitArgs 
         const u32x4 v = piece(kb, h);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const float f = ldexpf(bf16_bits_to_f32((v[j >> 1] >> (16 * (j & 1))) & 0xFFFFu), s);
+          const float f = scaled(v, j, s);
           const float g = rintf(f);
           // exact: f has 8 significant bits and |f - g| <= 1/2; a nonzero value
           // scaled into or below the subnormals counts as 2^-100
@@ -140,9 +167,31 @@ __global__ __launch_bounds__(kRdWaves * 64) void router_digits_kernel(DigitArgs 
   }
   res += __shfl_xor(res, 16, 64);
   res += __shfl_xor(res, 32, 64);
-  if (p == 0) wres[wave][r] = res;
+  if (p == 0) {
+    wres[wave][r] = res;
+    if (tok && res > 0.0f) atomicAdd(&large, (int)(16.0f * fminf(res, 1.0f)));
+  }
   __syncthreads();
+  const bool store = large > 16 * kRdResidue;  // tokens only
+  if (store) {
+    u32x4 *out = a.xr + (int64_t)blk * nk * 128 + lane;
+    for (int kb = kb0 + wave; kb < kb1; kb += kRdWaves)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u32x4 v = piece(kb, h);
+        u32x4 o = {0u, 0u, 0u, 0u};
+        if (!direct) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float f = scaled(v, j, s);
+            o[j >> 1] |= (__float_as_uint(f - rintf(f)) >> 16) << (16 * (j & 1));
+          }
+        }
+        out[(kb * 2 + h) * 64] = o;
+      }
+  }
   if (threadIdx.x < 16 && (int)threadIdx.x < rows) {  // wave 0: lane r holds row r's m and s
+    if (tok && r == 0) a.xflag[blk * 2 + blockIdx.y] = store;
     res = 0.0f;
 #pragma unroll
     for (int w = 0; w < kRdWaves; ++w) res += wres[w][r];
@@ -160,10 +209,10 @@ __global__ __launch_bounds__(kRdWaves * 64) void router_digits_kernel(DigitArgs 
 
 constexpr int kRdTok = 32;  // tokens of a workgroup's tile
 // Above this many open logits of its 1024 a workgroup takes its whole tile by
-// fp64 MFMA instead of one dot product a wave and logit: with one value of each
-// row 30000 times the others, 2048 tokens took 140 us by dot products, 112 with
-// the line at 256, 76 at 128 (the direct form 45).  At 300 times the dot products
-// stay the cheaper way (39 us), and ordinary rows leave a handful.
+// fp64 MFMA instead of one dot product a wave and logit: with every third of a
+// tile's logits open, 2048 tokens took 140 us by dot products, 112 with the line at
+// 256, 76 at 128.  Such tiles are those of rows that are not finite, and of
+// expert rows with a strong channel, whose residues are not stored.
 constexpr int kRdDense = 128;
 
 // A workgroup owns 32 tokens x 16 NJ experts, its waves the K blocks wave, wave
@@ -184,6 +233,8 @@ __global__ __launch_bounds__(256, OCC) void router_digits_mfma(DigitArgs a) {
   if (t0 >= a.T) return;
   const int nk = a.H / 64;
   if (threadIdx.x == 0) n_open = 0;
+  // byte 2 i + h: row block i of the tile stores the residues of half h
+  uint32_t flags = ldg<uint32_t>(reinterpret_cast<const uint32_t *>(a.xflag) + t0 / 32);
   const int8_t *ap[2], *bp[NJ];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -236,6 +287,77 @@ __global__ __launch_bounds__(256, OCC) void router_digits_mfma(DigitArgs a) {
 #pragma unroll
   for (int u = 0; u < D - 1; ++u)
     if (s + 4 * u < nk) multiply(u);
+  // The residues' products with w, where a row block has them: the wave's K blocks again.
+  const int r = lane & 15, q = lane >> 4;
+  const int kh = (nk + 1) / 2;
+  flags = __builtin_amdgcn_readfirstlane(flags) & (t0 + 16 < a.T ? 0x01010101u : 0x00000101u);
+  const bool residues = flags != 0;
+  auto stored = [&](int i, int h) { return (flags >> (16 * i + 8 * h) & 1u) != 0; };
+  f32x4 rs[OWN];  // of this wave's tiles
+#pragma unroll
+  for (int own = 0; own < OWN; ++own) rs[own] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (residues) {
+    f32x4 racc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) racc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint16_t *wr[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      wr[j] = a.w + (int64_t)min(e0 + 16 * j + r, a.E - 1) * a.H + 16 * q;
+    const u32x4 *xr[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      xr[i] = a.xr + (int64_t)min(t0 / 16 + i, (a.T - 1) / 16) * nk * 128 + lane;
+    constexpr int R = 3;  // K blocks in registers
+    u32x4 xv[R][2][2], wv[R][NJ][2];
+    auto fetch = [&](int slot, int kb) {  // past the end: the last block again, not used
+      kb = min(kb, nk - 1);
+      const int half = kb >= kh ? 1 : 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          xv[slot][i][h] = stored(i, half) ? ldg16(xr[i] + (kb * 2 + h) * 64)
+                                                                : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) wv[slot][j][h] = ldg16(wr[j] + kb * 64 + 8 * h);
+      }
+    };
+#pragma unroll
+    for (int d = 0; d < R - 1; ++d) fetch(d, wave + 4 * d);
+    int kb = wave;
+    while (kb < nk) {
+#pragma unroll
+      for (int u = 0; u < R; ++u, kb += 4) {
+        fetch((u + R - 1) % R, kb + 4 * (R - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        if (kb >= nk) continue;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+              racc[i * NJ + j] = BF16::mfma16x16x32(xv[u][i][h], wv[u][j][h], racc[i * NJ + j]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      if ((t & 3) != wave)
+        part[t & 3][wave - (wave > (t & 3) ? 1 : 0)][t >> 2][0][lane] =
+            __builtin_bit_cast(i32x4, racc[t]);
+    __syncthreads();
+#pragma unroll
+    for (int own = 0; own < OWN; ++own) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (wave == j) rs[own] = racc[4 * own + j];
+#pragma unroll
+      for (int o = 0; o < 3; ++o)
+        rs[own] = rs[own] + __builtin_bit_cast(f32x4, part[wave][o][own][0][lane]);
+    }
+    __syncthreads();  // part is used again below
+  }
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int owner = t & 3;
@@ -245,7 +367,6 @@ __global__ __launch_bounds__(256, OCC) void router_digits_mfma(DigitArgs a) {
       part[owner][wave - (wave > owner ? 1 : 0)][t >> 2][w][lane] = acc[t][w];
   }
   __syncthreads();
-  const int r = lane & 15, q = lane >> 4;
 #pragma unroll
   for (int own = 0; own < OWN; ++own) {
     // this wave's tile 4 own + wave
@@ -270,8 +391,19 @@ __global__ __launch_bounds__(256, OCC) void router_digits_mfma(DigitArgs a) {
       long long S = v[4][it];
 #pragma unroll
       for (int w = 3; w >= 0; --w) S = S * 256 + v[w][it];
-      const double L = ldexp((double)S, -(xt.s + we.s));
-      double eps = (((double)xt.r[0] + xt.r[1]) * we.m + ((double)we.r[0] + we.r[1]) * xt.m) * 1.001;
+      double L = ldexp((double)S, -(xt.s + we.s)), slack = 0.0;
+      double rx = (double)xt.r[0] + xt.r[1];
+      if (residues) {
+        const bool s0 = stored(i, 0), s1 = stored(i, 1);
+        rx = (s0 ? 0x1.0p-11 : 1.0) * xt.r[0] + (s1 ? 0x1.0p-11 : 1.0) * xt.r[1];
+        if ((s0 && xt.r[0] != 0.0f) || (s1 && xt.r[1] != 0.0f)) {
+          // L in 53 bits, values that count as 2^-100, products below the normal range; a sum
+          // that left fp32 opens the logit
+          L += ldexp((double)rs[own][it], -xt.s);
+          slack = fabs(L) * 0x1.0p-52 + ldexp(0x1.0p-87 * we.m + 0x1.0p-110, -xt.s) + 0.0 * rs[own][it];
+        }
+      }
+      double eps = (rx * we.m + ((double)we.r[0] + we.r[1]) * xt.m) * 1.001 + slack;
       if (S >= (1LL << 53) || S <= -(1LL << 53)) eps += fabs(L) * 0x1.0p-52;
       const float lo = round_bf16((float)(L - eps)), hi = round_bf16((float)(L + eps));
       if (lo == hi && (lo != 0.0f || eps == 0.0))  // an interval around 0 leaves the sign open
@@ -332,36 +464,48 @@ __global__ __launch_bounds__(256, OCC) void router_digits_mfma(DigitArgs a) {
   }
 }
 
-int64_t digit_bytes(int64_t rows, int64_t h) { return (rows + 15) / 16 * 16 * h * 3; }
-int64_t meta_bytes(int64_t rows) { return (rows + 15) / 16 * 16 * (int64_t)sizeof(RowMeta); }
+// Tokens per pass over the workspace, which bounds it (88 MB at H = 2048).
+constexpr int64_t kRdSlice = 8192;
+
+int64_t row_blocks(int64_t rows) { return (rows + 15) / 16; }
+int64_t digit_bytes(int64_t rows, int64_t h) { return row_blocks(rows) * 16 * h * 3; }
+int64_t meta_bytes(int64_t rows) { return row_blocks(rows) * 16 * (int64_t)sizeof(RowMeta); }
 
 }  // namespace
 
 int64_t router_digits_bytes(int64_t T, int64_t E, int64_t H) {
-  return digit_bytes(T, H) + digit_bytes(E, H) + meta_bytes(T) + meta_bytes(E);
+  T = std::min(T, kRdSlice);
+  return digit_bytes(T, H) + digit_bytes(E, H) + row_blocks(T) * 16 * H * 2 + meta_bytes(T) +
+         meta_bytes(E) + (T + 31) / 32 * 4;
 }
 
 int router_logits_digits(const uint16_t *x, const uint16_t *w, const float *bias, float *logits,
                          int64_t T, int64_t E, int64_t H, void *workspace, hipStream_t st) {
+  const int64_t slice = std::min(T, kRdSlice);
   DigitArgs a{};
-  a.x = x;
   a.w = w;
   a.bias = bias;
-  a.logits = logits;
-  int8_t *ws = static_cast<int8_t *>(workspace);
-  a.xd = ws;
-  a.wd = a.xd + digit_bytes(T, H);
-  a.xm = reinterpret_cast<RowMeta *>(a.wd + digit_bytes(E, H));
-  a.wm = reinterpret_cast<RowMeta *>(reinterpret_cast<int8_t *>(a.xm) + meta_bytes(T));
-  a.T = (int)T;
+  a.xd = static_cast<int8_t *>(workspace);
+  a.wd = a.xd + digit_bytes(slice, H);
+  a.xr = reinterpret_cast<u32x4 *>(a.wd + digit_bytes(E, H));
+  a.xm = reinterpret_cast<RowMeta *>(a.xr + row_blocks(slice) * H * 2);
+  a.wm = a.xm + row_blocks(slice) * 16;
+  a.xflag = reinterpret_cast<uint8_t *>(a.wm + row_blocks(E) * 16);
   a.E = (int)E;
   a.H = (int)H;
-  router_digits_kernel<<<dim3(cdiv(T, 16) + cdiv(E, 16), 2), kRdWaves * 64, (size_t)H * 32, st>>>(a);
-  if (int rc = check_launch("router_digits_kernel")) return rc;
-  constexpr int NJ = 2;  // 32 x 32 logits, two workgroups per CU (4, one per CU: no faster)
-  const unsigned grid = 8 * cdiv(cdiv(T, kRdTok), 8) * cdiv(E, 16 * NJ);
-  router_digits_mfma<NJ, 2><<<grid, 256, 0, st>>>(a);
-  return check_launch("router_digits_mfma");
+  for (int64_t t = 0; t < T; t += slice) {
+    a.x = x + t * H;
+    a.logits = logits + t * E;
+    a.T = (int)std::min(slice, T - t);
+    const unsigned blocks = cdiv(a.T, 16) + (t ? 0 : cdiv(E, 16));  // the weights once
+    router_digits_kernel<<<dim3(blocks, 2), kRdWaves * 64, (size_t)H * 32, st>>>(a);
+    if (int rc = check_launch("router_digits_kernel")) return rc;
+    constexpr int NJ = 2;  // 32 x 32 logits, two workgroups per CU (4, one per CU: no faster)
+    const unsigned grid = 8 * cdiv(cdiv(a.T, kRdTok), 8) * cdiv(E, 16 * NJ);
+    router_digits_mfma<NJ, 2><<<grid, 256, 0, st>>>(a);
+    if (int rc = check_launch("router_digits_mfma")) return rc;
+  }
+  return LM_OK;
 }
 
 }  // namespace lm

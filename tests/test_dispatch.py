@@ -53,3 +53,10 @@ def test_short_last_row_tile_stays_with_its_columns():
     by columns two rounds (36)."""
     assert linear_form(1060, 4096, 2048) == (STREAMED, 128, 128, 0)
     assert linear_form(1280, 4096, 2048) == (STREAMED, 128, 128, 1)
+
+
+def test_router_workspace_is_bounded():
+    """Calls of many tokens pass over one workspace in slices."""
+    need = _lib.lib().lm_router_workspace_bytes
+    assert 0 < need(2048, 256, 2048) < need(8192, 256, 2048) == need(65536, 256, 2048) < 100 << 20
+    assert need(65536, 256, 4096) == need(1 << 20, 256, 4096) < 200 << 20

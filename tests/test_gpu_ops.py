@@ -459,6 +459,69 @@ def test_router_digits(dev, t, e, h, kind):
         assert torch.equal(got[1][fine].view(torch.int16), ref[1][fine].view(torch.int16))
 
 
+def _digit_router(x, w, k, bias=None):
+    """router_topk through the int8-digit form, whatever its size."""
+    t, h = x.shape
+    e = w.shape[0]
+    need = _lib.lib().lm_router_workspace_bytes(t, e, h)
+    assert need > 0
+    lg = torch.empty(t, e, device=x.device)
+    ids = torch.empty(t, k, dtype=torch.int64, device=x.device)
+    wts = torch.empty(t, k, dtype=torch.bfloat16, device=x.device)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    _lib.call('lm_router_topk_ws', x.data_ptr(), w.data_ptr(), _lib.ptr(bias), lg.data_ptr(),
+              ids.data_ptr(), wts.data_ptr(), t, e, h, k, ws.data_ptr(), need,
+              _lib.stream(x.device))
+    return lg, wts, ids
+
+
+@pytest.mark.parametrize('t,e,h', [(513, 256, 2048), (1000, 200, 768), (530, 17, 256),
+                                   (600, 100, 4096), (8192 + 40, 40, 512)])
+@pytest.mark.parametrize('kind', ['normal', 'channel', 'half', 'few rows', 'weights', 'range',
+                                  'small', 'large'])
+def test_router_digit_residues(dev, t, e, h, kind):
+    """Rows whose residues are stored (a strong channel of all rows, of a half of
+    the row blocks, of a few rows; values of a wide range; tiny and huge ones, so
+    that scaled values or sums leave the normal range) against the fp64 form, bit
+    for bit, among rows of zeros, infinities and NaN and in a second slice of tokens."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(t)
+    x = torch.randn(t, h, generator=g, device=dev)
+    w = torch.randn(e, h, generator=g, device=dev) * 0.02
+    if kind == 'channel':
+        x[:, 77] *= 20000
+    if kind == 'half':
+        x[(torch.arange(t, device=dev) // 16) % 2 == 0, h - 3] *= 5000
+    if kind == 'few rows':
+        x[::41, 5] *= 1e5
+    if kind == 'weights':
+        x[:, 3] *= 3000
+        w[::3, 9] *= 3000
+    if kind == 'range':
+        x = x * torch.exp2(torch.randint(-60, 31, (t, h), generator=g, device=dev).float())
+    if kind == 'small':
+        x, w = x * 1e-25, w * 1e-10
+        x[:, 77] *= 3000
+    if kind == 'large':
+        x, w = x * 1e32, w * 1e5
+        x[:, 77] *= 3000
+    x[7] = 0
+    x[11] *= 1e-37
+    x[20, 1] = float('inf')
+    x[t - 1, 2] = float('nan')
+    w[e // 2, 5] = float('-inf')
+    w[1] *= 1e-35
+    x, w = x.to(torch.bfloat16), w.to(torch.bfloat16)
+    got, ref = _digit_router(x, w, 4), _direct_router(x, w, 4, None)
+    nan = ref[0].isnan()
+    assert torch.equal(got[0].isnan(), nan)
+    assert torch.equal(got[0].view(torch.int32).where(~nan, 0),
+                       ref[0].view(torch.int32).where(~nan, 0))
+    fine = ~nan.any(-1)
+    assert torch.equal(got[2][fine], ref[2][fine])
+    assert torch.equal(got[1][fine].view(torch.int16), ref[1][fine].view(torch.int16))
+
+
 def test_rmsnorm_bit_exact(dev):
     gen = seeded(11)
     x = bf16_rand((5, 2048), gen, 3.0)
