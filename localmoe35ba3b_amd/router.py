@@ -31,7 +31,12 @@ def router_topk(hidden, weight, top_k, bias=None):
     if bias is not None:
         bias = bias.to(device=dev, dtype=torch.float32).contiguous()
     need = _lib.lib().lm_router_workspace_bytes(tokens, experts, h)
-    workspace = hidden.new_empty(need, dtype=torch.uint8) if need else None
+    workspace = None
+    if need:
+        try:
+            workspace = hidden.new_empty(need, dtype=torch.uint8)
+        except torch.OutOfMemoryError:
+            need = 0  # without a workspace: the same values, in more time
     _lib.call('lm_router_topk_ws', hidden.data_ptr(), weight.contiguous().data_ptr(),
               _lib.ptr(bias), logits.data_ptr(), ids.data_ptr(), weights.data_ptr(), tokens,
               experts, h, top_k, _lib.ptr(workspace), need, _lib.stream(dev))

@@ -3,7 +3,7 @@ refused, and replaced module-level operators are called.  Tensors that only clai
 import pytest
 import torch
 
-from localmoe35ba3b_amd import _lib
+from localmoe35ba3b_amd import _lib, router
 from localmoe35ba3b_amd.operators import int8, w8a8
 
 
@@ -83,3 +83,19 @@ def test_experts_call_replaced_operators(launches, monkeypatch, name):
     assert calls == [name] * (2 if name == 'grouped_linear' else 1)
     assert launches[1:] == ['lm_expert_table', 'lm_w8a16_grouped_gemv', 'lm_swiglu',
                             'lm_w8a16_grouped_gemv', 'lm_ordered_reduce']
+
+
+def test_router_without_memory_for_its_workspace(launches, monkeypatch):
+    """A router call that finds no memory for its scratch runs the form without."""
+    new_empty, args = torch.Tensor.new_empty, []
+
+    def full(self, size, dtype=None, **kw):
+        if dtype is torch.uint8:
+            raise torch.OutOfMemoryError('no memory')
+        return new_empty(self, size, dtype=dtype or self.dtype, **kw)
+
+    monkeypatch.setattr(OnGpu, 'new_empty', full)
+    monkeypatch.setattr(_lib, 'call', lambda name, *a: args.append((name, a[-3:-1])))
+    router.router_topk(gpu(torch.zeros(2048, 2048, dtype=torch.bfloat16)),
+                       gpu(torch.zeros(256, 2048, dtype=torch.bfloat16)), 8)
+    assert args == [('lm_router_topk_ws', (None, 0))]
