@@ -295,11 +295,13 @@ int lm_router_topk(const void *x, const void *w, const float *bias,
 
 /* lm_router_topk with device scratch of the caller, for calls of many tokens,
  * whose logits are then taken from exact int8 products (the same logits, ids
- * and weights, faster).  lm_router_workspace_bytes says how much the call
- * takes (0: the call uses none); workspace is 16-byte aligned, NULL runs
- * lm_router_topk, a smaller one than stated is LM_ENOMEM.  Every byte read is
- * written by the call first.  No counterpart in the reference (HF:768-776). */
+ * and weights).  lm_router_workspace_bytes says how much the call takes (0: the
+ * call uses none), lm_router_workspace_pays whether it is faster with it (1) or
+ * without (0); workspace is 16-byte aligned, NULL runs lm_router_topk, a smaller
+ * one than stated is LM_ENOMEM.  Every byte used is written by the call first.
+ * No counterpart in the reference (HF:768-776). */
 int64_t lm_router_workspace_bytes(int64_t tokens, int64_t experts, int64_t hidden);
+int lm_router_workspace_pays(int64_t tokens, int64_t experts, int64_t hidden);
 int lm_router_topk_ws(const void *x, const void *w, const float *bias,
                       float *logits, int64_t *ids, void *weights,
                       int64_t tokens, int64_t experts, int64_t hidden,

@@ -58,6 +58,7 @@ SIGNATURES = {
                                        I64, I64, I32, P]),
     'lm_router_topk': (I32, [P, P, P, P, P, P, I64, I64, I64, I64, P]),
     'lm_router_workspace_bytes': (I64, [I64, I64, I64]),
+    'lm_router_workspace_pays': (I32, [I64, I64, I64]),
     'lm_router_topk_ws': (I32, [P, P, P, P, P, P, I64, I64, I64, I64, P, I64, P]),
     'lm_rmsnorm': (I32, [P, P, P, I64, I64, F32, P]),
     'lm_moe_workspace_bytes': (I64, [I64, I64, I64, I64, I64]),

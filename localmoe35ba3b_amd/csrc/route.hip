@@ -197,6 +197,23 @@ static bool router_digits_serves(int64_t T, int64_t H) {
   return T > kDigitTokens && H % 256 == 0 && H <= 4096;
 }
 
+// Whether the digits are the faster form, by estimates in us fitted over 480
+// sizes of 513 to 16384 tokens, 16 to 256 experts and hidden 256 to 4096, where
+// the choice is 0.1 % slower than the better of both.  The fp64 tiles cost their
+// rounds of 16 x 32 on 256 CUs, the digits two launches and their passes, so few
+// experts or a short row leave nothing to gain: 2048 tokens and 256 experts take
+// 32 us against 46 at hidden 2048, 23 against 27 at 1024, 16 against 13 at 256; 32
+// experts at 2048 hidden 26 against 12.  The margin is for rows with large
+// residues, which cost the digits up to a third more.
+static bool router_digits_pay(int64_t T, int64_t E, int64_t H) {
+  const double h = (double)H / 1024.0;
+  const int64_t tiles = ((T + 15) / 16) * ((E + 31) / 32);
+  const double fp64 = 7.0 + 4.75 * h * (double)((tiles + 255) / 256);
+  const double more = (double)std::max<int64_t>(T - 1024, 0) / 1024.0;
+  const double digits = 12.0 + 4.2 * h + more * (0.8 + h * (1.75 + 0.0085 * (double)E));
+  return H >= 512 && fp64 > 1.05 * digits;
+}
+
 int router_topk(const float *logits, int64_t T, int64_t E, int64_t K, int64_t *ids,
                 uint16_t *weights, hipStream_t st) {
   topk_kernel<<<cdiv(T, 4), 256, 0, st>>>(logits, (int)T, (int)E, (int)K, ids, weights);
@@ -525,6 +542,11 @@ using namespace lm;
 extern "C" int64_t lm_router_workspace_bytes(int64_t tokens, int64_t experts, int64_t hidden) {
   if (experts < 1 || experts > 256 || hidden < 1 || !router_digits_serves(tokens, hidden)) return 0;
   return router_digits_bytes(tokens, experts, hidden);
+}
+
+extern "C" int lm_router_workspace_pays(int64_t tokens, int64_t experts, int64_t hidden) {
+  return lm_router_workspace_bytes(tokens, experts, hidden) > 0 &&
+         router_digits_pay(tokens, experts, hidden);
 }
 
 extern "C" int lm_router_topk_ws(const void *x, const void *w, const float *bias, float *logits,

@@ -30,9 +30,9 @@ def router_topk(hidden, weight, top_k, bias=None):
     weights = hidden.new_empty((tokens, top_k))
     if bias is not None:
         bias = bias.to(device=dev, dtype=torch.float32).contiguous()
-    need = _lib.lib().lm_router_workspace_bytes(tokens, experts, h)
-    workspace = None
-    if need:
+    lib, need, workspace = _lib.lib(), 0, None
+    if lib.lm_router_workspace_pays(tokens, experts, h):
+        need = lib.lm_router_workspace_bytes(tokens, experts, h)
         try:
             workspace = hidden.new_empty(need, dtype=torch.uint8)
         except torch.OutOfMemoryError:

@@ -60,3 +60,15 @@ def test_router_workspace_is_bounded():
     need = _lib.lib().lm_router_workspace_bytes
     assert 0 < need(2048, 256, 2048) < need(8192, 256, 2048) == need(65536, 256, 2048) < 100 << 20
     assert need(65536, 256, 4096) == need(1 << 20, 256, 4096) < 200 << 20
+
+
+def test_router_digits_only_where_they_pay():
+    """Few experts, a short row or few tokens keep the fp64 tiles, which take
+    half the time there."""
+    pays = _lib.lib().lm_router_workspace_pays
+    for t, e, h in ((513, 256, 2048), (2048, 256, 2048), (65536, 256, 2048), (2048, 256, 4096),
+                    (4096, 256, 1024), (16384, 128, 2048)):
+        assert pays(t, e, h), (t, e, h)
+    for t, e, h in ((512, 256, 2048), (1024, 128, 2048), (16384, 17, 2048), (65536, 16, 4096),
+                    (16384, 256, 256), (600, 256, 512), (2048, 256, 2016), (2048, 256, 8192)):
+        assert not pays(t, e, h), (t, e, h)
