@@ -464,9 +464,14 @@ __global__ __launch_bounds__(256, OCC) void router_digits_mfma(DigitArgs a) {
   }
 }
 
-// Tokens per pass over the workspace, which bounds it (88 MB at H = 2048).
-constexpr int64_t kRdSlice = 8192;
-
+// Tokens per pass over the workspace, which bounds it (336 MB): as few passes as
+// do, of whole tiles and about the same size.  Each further one costs its launches and a
+// last round (20000 tokens: 152 us in one pass, 183 in three).
+int64_t slice_tokens(int64_t T, int64_t H) {
+  const int64_t most = (int64_t(64) << 20) / H;
+  const int64_t passes = (T + most - 1) / most;
+  return std::min(most, ((T + passes - 1) / passes + 31) / 32 * 32);
+}
 int64_t row_blocks(int64_t rows) { return (rows + 15) / 16; }
 int64_t digit_bytes(int64_t rows, int64_t h) { return row_blocks(rows) * 16 * h * 3; }
 int64_t meta_bytes(int64_t rows) { return row_blocks(rows) * 16 * (int64_t)sizeof(RowMeta); }
@@ -474,14 +479,14 @@ int64_t meta_bytes(int64_t rows) { return row_blocks(rows) * 16 * (int64_t)sizeo
 }  // namespace
 
 int64_t router_digits_bytes(int64_t T, int64_t E, int64_t H) {
-  T = std::min(T, kRdSlice);
+  T = std::min(T, (int64_t(64) << 20) / H);
   return digit_bytes(T, H) + digit_bytes(E, H) + row_blocks(T) * 16 * H * 2 + meta_bytes(T) +
          meta_bytes(E) + (T + 31) / 32 * 4;
 }
 
 int router_logits_digits(const uint16_t *x, const uint16_t *w, const float *bias, float *logits,
                          int64_t T, int64_t E, int64_t H, void *workspace, hipStream_t st) {
-  const int64_t slice = std::min(T, kRdSlice);
+  const int64_t slice = slice_tokens(T, H);
   DigitArgs a{};
   a.w = w;
   a.bias = bias;

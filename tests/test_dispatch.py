@@ -58,8 +58,8 @@ def test_short_last_row_tile_stays_with_its_columns():
 def test_router_workspace_is_bounded():
     """Calls of many tokens pass over one workspace in slices."""
     need = _lib.lib().lm_router_workspace_bytes
-    assert 0 < need(2048, 256, 2048) < need(8192, 256, 2048) == need(65536, 256, 2048) < 100 << 20
-    assert need(65536, 256, 4096) == need(1 << 20, 256, 4096) < 200 << 20
+    assert 0 < need(2048, 256, 2048) < need(32768, 256, 2048) == need(65536, 256, 2048)
+    assert need(16384, 256, 4096) == need(65536, 256, 4096) == need(1 << 20, 256, 4096) < 336 << 20
 
 
 def test_router_digits_only_where_they_pay():
