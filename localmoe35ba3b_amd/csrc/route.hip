@@ -417,10 +417,11 @@ __global__ __launch_bounds__(256) void ordered_reduce_kernel(const uint16_t *__r
 // prefill._reduce: per token, routes in ascending expert order, rounding to
 // T at every step.  Routes are clamped into [0, tokens * K), slots into [0, K).
 // A thread owns VEC adjacent columns (one 16-byte load per route at VEC = 8)
-// and requests the rows of eight routes before it adds the first, so a token
-// of 8 routes costs one index latency and one row latency; with 2-byte loads
-// route by route the 75 MB of 2048 tokens x 8 took 58 us, now 18 us (8192
-// tokens: 282 against 52 us, 5.8 TB/s).
+// and requests the rows of B routes before it adds the first.  Two are enough with
+// the many waves of a call, and fewer registers and repeated rows than eight:
+// 2048 tokens x 8 routes x 2048 columns take 57 us with 2-byte loads route by
+// route, 17.6 with eight in flight, 14.2 with two (8192 tokens 274, 49 and 50 us,
+// 6 TB/s); one route of 4096 columns 20.8, 14.1 and 7.5.
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void routed_reduce_kernel(const uint16_t *__restrict__ v,
                                                             const int64_t *__restrict__ ordered,
@@ -428,7 +429,7 @@ __global__ __launch_bounds__(256) void routed_reduce_kernel(const uint16_t *__re
                                                             const void *w, int w_dtype,
                                                             uint16_t *__restrict__ y, int N,
                                                             int K, int64_t routes) {
-  constexpr int B = 8;  // routes per batch
+  constexpr int B = VEC == 8 ? 2 : 1;  // routes per batch
   const int tok = blockIdx.y;
   const int n = (blockIdx.x * blockDim.x + threadIdx.x) * VEC;
   if (n >= N) return;
@@ -474,9 +475,11 @@ template <typename T>
 static int routed_reduce(const uint16_t *v, const int64_t *ordered, const int64_t *slots,
                          const void *w, int w_dtype, uint16_t *y, int64_t tokens, int64_t n,
                          int64_t top_k, hipStream_t st) {
-  // whole 16-byte pieces where the rows allow them, else one column a thread
-  const bool wide =
-      n % 8 == 0 && ((reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
+  // whole 16-byte pieces where the rows allow them, else one column a thread; rows of
+  // fewer than 256 columns too, whose pieces fill no wave (16 routes of 128 columns, 300
+  // tokens: 6.5 us, with pieces 9.0)
+  const bool wide = n >= 256 && n % 8 == 0 &&
+                    ((reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
   const int64_t threads = wide ? n / 8 : n;
   const unsigned block = threads <= 64 ? 64 : threads <= 128 ? 128 : 256;
   const dim3 grid(cdiv(threads, block), (unsigned)tokens);

@@ -476,7 +476,7 @@ def _digit_router(x, w, k, bias=None):
 
 
 @pytest.mark.parametrize('t,e,h', [(513, 256, 2048), (1000, 200, 768), (530, 17, 256),
-                                   (600, 100, 4096), (8192 + 40, 40, 512)])
+                                   (600, 100, 4096), (16384 + 40, 17, 4096)])
 @pytest.mark.parametrize('kind', ['normal', 'channel', 'half', 'few rows', 'weights', 'range',
                                   'small', 'large'])
 def test_router_digit_residues(dev, t, e, h, kind):
@@ -663,6 +663,23 @@ def test_routed_reduce_forms(dev, k, n, off):
     _, _, ro, rs = O.plan(ids.numpy(), e, 96)
     for tok in range(t):
         ref = O.ordered_combine(npf(v)[ro[tok]], npf(w)[tok, rs[tok]], O.bf16)
+        assert np.array_equal(npf(y[tok]), ref)
+
+
+@pytest.mark.parametrize('k', [1, 2, 3, 7, 16])
+@pytest.mark.parametrize('n', [248, 256, 264])
+def test_routed_reduce_batches(dev, k, n):
+    """Odd and even route counts around the narrowest rows of 16-byte pieces."""
+    t, e = 5, 40
+    ids = _ids(seeded(k + n), t, e, k, False)
+    _, _, ordered, slots = gpu_routes.plan(ids.to(dev), e, 96)
+    gen = seeded(53)
+    v = (torch.randn(t * k, n, generator=gen) * 2).to(torch.float16)
+    w = torch.softmax(torch.randn(t, k, generator=gen), -1)
+    y = gpu_routes.routed_reduce(v.to(dev), ordered, slots, w.to(dev), t, n)
+    _, _, ro, rs = O.plan(ids.numpy(), e, 96)
+    for tok in range(t):
+        ref = O.ordered_combine(npf(v)[ro[tok]], w.numpy()[tok, rs[tok]], O.fp16)
         assert np.array_equal(npf(y[tok]), ref)
 
 
