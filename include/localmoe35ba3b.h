@@ -460,6 +460,18 @@ int lm_moe_layer_forward_chain(const lm_moe_layer *layer,
                                void *weights_out, void *const *phase_events,
                                void *stream);
 
+/* lm_moe_layer_forward_chain for a chunk that runs at the same time as others on
+ * further streams, the largest of beside_tokens: its GEMMs take the form that is
+ * faster beside that one.  The results are the same for any value. */
+int lm_moe_layer_forward_beside(const lm_moe_layer *layer,
+                                const lm_moe_layer *next, int input_normed,
+                                int64_t beside_tokens, void *h, int64_t tokens,
+                                int64_t hidden, int64_t inter, int64_t experts,
+                                int64_t top_k, float eps, void *workspace,
+                                int64_t workspace_bytes, int32_t *ids_out,
+                                void *weights_out, void *const *phase_events,
+                                void *stream);
+
 /* lm_moe_layer_forward without a workspace argument: the call's workspace
  * is a device array inside the library (one per device, about 7.3 MB, held
  * until the process ends), so the call allocates nothing and takes no

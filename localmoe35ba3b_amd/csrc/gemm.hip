@@ -920,8 +920,13 @@ constexpr int64_t kDenseTallM = 1024;
 // Few rows per expert (a short prompt, a small batch): gate_up on the tile
 // layout takes 32 columns per wave at 3 workgroups per CU and the deep rings
 // instead: 26 -> 17 us at 2 tokens, 66 -> 53 at 24, 110 -> 95 at 256, 117 ->
-// 111 at 1024 (256 experts, top-8).  Above that a chunk overlaps with another one,
-// where the 64-column form is faster (above).
+// 111 at 1024 (256 experts, top-8; a layer of 16 unskewed tokens, whose 103 experts
+// then take a second round, 88 -> 92, and of 56 to 128 1 % more).  Above that a chunk
+// overlaps with another one, where the 64-column form is faster (above), and so it is for
+// a short chunk beside such a one: 1024 tokens beside 2048 in three layers 1240
+// -> 1208 us, 256 skewed ones 932 -> 906.  Chunks of up to 1024 tokens beside
+// each other keep the 32 columns (256: 0.96 to 1.01 of the time, 512 0.97 to 1.01, 1024
+// 0.97 to 1.03).
 constexpr int64_t kFewRows = 36;
 // Wide dense tiles: 8 waves over 256 columns of a 128-row tile, one
 // workgroup per CU.  Each activation stage then feeds twice the columns, a
@@ -1154,7 +1159,7 @@ int routed_gemm(const RoutedGemm &r, hipStream_t st) {
   a.N = (int)r.n;
   a.K = (int)r.k;
   a.tile_rows = (int)r.bm;
-  a.few_rows = r.y_rows <= kFewRows * r.experts;
+  a.few_rows = std::max(r.y_rows, r.form_rows) <= kFewRows * r.experts;
   const unsigned mt = (unsigned)r.n_tiles;
   return r.dtype == LM_BF16 ? routed_dispatch<BF16>(a, mt, r.gather, r.swiglu, st)
                             : routed_dispatch<FP16>(a, mt, r.gather, r.swiglu, st);

@@ -40,6 +40,9 @@ struct RoutedGemm {
   // ptile[i * bm + r] (any value for rows past the tile's end), read with the
   // table row instead of through pos; required with q_tiles and gather.
   const int *ptile = nullptr;
+  // Output rows that choose the tile form where another call's GEMM runs at the
+  // same time and has more rows (results are the same); 0: y_rows.
+  int64_t form_rows = 0;
 };
 int routed_gemm(const RoutedGemm &r, hipStream_t st);
 

@@ -1491,9 +1491,10 @@ int check_layer(const lm_moe_layer *layer) {
 // also leaves next's normalized inputs for the same rows in the workspace;
 // with input_normed, the workspace already holds this layer's (a chained
 // call before it) and the norm kernel is not launched.  Decode calls ignore
-// both: their router kernel normalizes the row itself.
+// both: their router kernel normalizes the row itself.  beside_tokens: tokens of the
+// largest call that runs at the same time.
 int layer_forward(const lm_moe_layer *layer, const lm_moe_layer *next, bool input_normed,
-                  void *h, int64_t tokens, int64_t hidden, int64_t inter, int64_t experts,
+                  int64_t beside_tokens, void *h, int64_t tokens, int64_t hidden, int64_t inter, int64_t experts,
                   int64_t top_k, float eps, void *workspace, int64_t workspace_bytes,
                   int32_t *ids_out, void *weights_out, void *const *phase_events, void *stream) {
   LM_REQUIRE(hidden == kH && inter == kI && experts == kE && top_k == kTopK, LM_EINVAL,
@@ -1619,7 +1620,8 @@ int layer_forward(const lm_moe_layer *layer, const lm_moe_layer *next, bool inpu
   const RoutedGemm gu{f16 ? a.xh : a.xn, kH,  T,  a.gu_q, a.gu_s,  a.gu_qes, a.gu_ses,
                       kE + 1,  pos,     table, w.n_tiles, kBM, a.hbuf, R + T,
                       2 * kI,  kH,      true,  true,   LM_BF16, layer->gu_q_tiles,
-                      f16 ? a.xk : nullptr, ptile};
+                      f16 ? a.xk : nullptr, ptile,
+                      std::min<int64_t>(beside_tokens, 65536) * (kTopK + 1)};
   if (int rc = routed_gemm(gu, st)) return rc;
   if (int rc = mark(5)) return rc;
   const RoutedGemm dn{a.hbuf,  kI,      R + T, a.dn_q, a.dn_s, a.dn_qes, a.dn_ses,
@@ -1648,7 +1650,7 @@ extern "C" int lm_moe_layer_forward(const lm_moe_layer *layer, void *h, int64_t 
                                     float eps, void *workspace, int64_t workspace_bytes,
                                     int32_t *ids_out, void *weights_out,
                                     void *const *phase_events, void *stream) {
-  return layer_forward(layer, nullptr, false, h, tokens, hidden, inter, experts, top_k, eps,
+  return layer_forward(layer, nullptr, false, 0, h, tokens, hidden, inter, experts, top_k, eps,
                        workspace, workspace_bytes, ids_out, weights_out, phase_events, stream);
 }
 
@@ -1659,9 +1661,22 @@ extern "C" int lm_moe_layer_forward_chain(const lm_moe_layer *layer, const lm_mo
                                           int64_t workspace_bytes, int32_t *ids_out,
                                           void *weights_out, void *const *phase_events,
                                           void *stream) {
-  return layer_forward(layer, next, input_normed != 0, h, tokens, hidden, inter, experts, top_k,
-                       eps, workspace, workspace_bytes, ids_out, weights_out, phase_events,
+  return layer_forward(layer, next, input_normed != 0, 0, h, tokens, hidden, inter, experts,
+                       top_k, eps, workspace, workspace_bytes, ids_out, weights_out, phase_events,
                        stream);
+}
+
+extern "C" int lm_moe_layer_forward_beside(const lm_moe_layer *layer, const lm_moe_layer *next,
+                                           int input_normed, int64_t beside_tokens, void *h,
+                                           int64_t tokens, int64_t hidden, int64_t inter,
+                                           int64_t experts, int64_t top_k, float eps,
+                                           void *workspace, int64_t workspace_bytes,
+                                           int32_t *ids_out, void *weights_out,
+                                           void *const *phase_events, void *stream) {
+  LM_REQUIRE(beside_tokens >= 0, LM_EINVAL, "invalid token count");
+  return layer_forward(layer, next, input_normed != 0, beside_tokens, h, tokens, hidden, inter,
+                       experts, top_k, eps, workspace, workspace_bytes, ids_out, weights_out,
+                       phase_events, stream);
 }
 
 extern "C" int64_t lm_moe_static_max_tokens(void) { return kScratchMaxTokens; }

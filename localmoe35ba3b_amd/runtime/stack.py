@@ -170,9 +170,10 @@ class MoEStack:
         return ws
 
     def layer_forward(self, h, l, ids_out=None, weights_out=None, events=None, workspace=None,
-                      next_layer=None, input_normed=False):
+                      next_layer=None, input_normed=False, beside=0):
         """h bf16 [T, H] updated in place: h = h + block(rmsnorm(h)).  Chunks
-        in flight at the same time need workspaces of their own.
+        in flight at the same time need workspaces of their own; beside, the
+        tokens of the largest other one, only chooses the faster tiles.
 
         Chained calls (lm_moe_layer_forward_chain): with next_layer, the call
         also leaves layer next_layer's normalized inputs for these rows in the
@@ -189,16 +190,17 @@ class MoEStack:
         if events is not None:
             ev = (ctypes.c_void_p * len(events))(*[e.cuda_event for e in events])
         ws = self.workspace if workspace is None else workspace
-        if next_layer is None and not input_normed:
+        if next_layer is None and not input_normed and not beside:
             _lib.call('lm_moe_layer_forward', ctypes.byref(self._structs[l]), h.data_ptr(), tokens,
                       self.H, self.I, self.E, self.K, EPS, ws.data_ptr(), ws.numel(),
                       _lib.ptr(ids_out), _lib.ptr(weights_out), ev, _lib.stream(h.device))
             return h
         nxt = None if next_layer is None else ctypes.byref(self._structs[next_layer])
-        _lib.call('lm_moe_layer_forward_chain', ctypes.byref(self._structs[l]), nxt,
-                  int(bool(input_normed)), h.data_ptr(), tokens, self.H, self.I, self.E, self.K,
-                  EPS, ws.data_ptr(), ws.numel(), _lib.ptr(ids_out), _lib.ptr(weights_out), ev,
-                  _lib.stream(h.device))
+        name, extra = (('lm_moe_layer_forward_beside', (beside,)) if beside else
+                       ('lm_moe_layer_forward_chain', ()))
+        _lib.call(name, ctypes.byref(self._structs[l]), nxt, int(bool(input_normed)), *extra,
+                  h.data_ptr(), tokens, self.H, self.I, self.E, self.K, EPS, ws.data_ptr(),
+                  ws.numel(), _lib.ptr(ids_out), _lib.ptr(weights_out), ev, _lib.stream(h.device))
         return h
 
     _REGION_TYPES = {'normed': (torch.bfloat16, 'H'), 'gate': (torch.float32, None),
@@ -316,7 +318,7 @@ class MoEStack:
                         st.wait_event(done[c - 1][l - 1])
                     self.layer_forward(h[c0:c0 + chunk], l, workspace=spaces[c % 2],
                                        next_layer=l + 1 if chain and l + 1 < self.L else None,
-                                       input_normed=chain and l > 0)
+                                       input_normed=chain and l > 0, beside=chunk)
                     done[c][l].record(st)
         cur.wait_stream(self._side)
         self._done_events = done  # kept alive until the next call

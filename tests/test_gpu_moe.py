@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 import torch
 
-from localmoe35ba3b_amd import router
+from localmoe35ba3b_amd import _lib, router
 from localmoe35ba3b_amd.runtime.stack import EPS, SyntheticMoEStack, zipf_bias
 from oracle import moe_oracle as O
 from tests.conftest import BF16_TOL, assert_close
@@ -375,6 +375,28 @@ def test_chained_layers_bit_identical(dev, fmt, tokens):
     if tokens > 1:
         two = st.prefill(h, chunk=(tokens + 1) // 2, overlap=True)  # two chained chunks
         assert torch.equal(two, plain)
+
+
+@pytest.mark.parametrize('fmt', [0, 1])
+def test_beside_chooses_tiles_only(dev, fmt):
+    """A chunk that runs beside a larger one takes that one's tile form, with the
+    same bits, and overlapped prefill says which chunk that is."""
+    st = SyntheticMoEStack(layers=2, seed=43, device=dev, max_tokens=1600, gate_up_format=fmt)
+    x = inputs(1700, 44, dev)
+    alone = st.forward(x[1600:].clone())
+    h = x[1600:].clone()
+    st.layer_forward(h, 0, next_layer=1, beside=1600)
+    st.layer_forward(h, 1, input_normed=True, beside=1600)
+    assert torch.equal(h, alone)
+    with pytest.raises(ValueError, match='token count'):
+        st.layer_forward(h, 0, beside=-1)
+    calls, call = [], _lib.call
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(_lib, 'call', lambda *a: calls.append(a) or call(*a))
+        out = st.prefill(x, chunk=1600)
+    assert torch.equal(out[1600:], alone)
+    assert [(a[0], a[4]) for a in calls if 'forward' in a[0]] == [
+        ('lm_moe_layer_forward_beside', 1600)] * 4
 
 
 def test_tile_copy_stale_weights_refused(dev):
