@@ -928,6 +928,10 @@ constexpr int64_t kDenseTallM = 1024;
 // each other keep the 32 columns (256: 0.96 to 1.01 of the time, 512 0.97 to 1.01, 1024
 // 0.97 to 1.03).
 constexpr int64_t kFewRows = 36;
+// The same on the standard layout, which has 32 columns per wave in any case, so
+// that only the rings differ: gate_up 57 -> 50 us at 24 tokens, 109 -> 98 at 256, 113
+// -> 108 at 600, but 115 -> 118 at 800 and 121 -> 128 at 1024.
+constexpr int64_t kFewRowsPlain = 21;
 // Wide dense tiles: 8 waves over 256 columns of a 128-row tile, one
 // workgroup per CU.  Each activation stage then feeds twice the columns, a
 // third fewer wave-loads per MFMA than two 4-wave workgroups; taken when the
@@ -947,7 +951,8 @@ static int launch_rb(GemmArgs a, unsigned mtiles, hipStream_t st) {
   constexpr int AD = TALL ? kRbADTall : kRbAD;
   // gate_up at 32 columns per wave; the down GEMM's 8 stages are no longer
   // than the deep ring, which made it slower (33 -> 39 us at 24 tokens)
-  constexpr bool DEEP = K == 2048 && WL != kWlDirect && TN == kRbTN;
+  constexpr bool DEEP = K == 2048 && FEW;
+  static_assert(!DEEP || (WL != kWlDirect && TN == kRbTN), "deep rings serve routed rows");
   constexpr int RBN = NW * TN;
   a.nt_count = SWIGLU ? (int)cdiv(a.N / 2, RBN / 2) : (int)cdiv(a.N, RBN);
   a.mt_count = (int)mtiles;
@@ -976,8 +981,8 @@ static int launch_grouped(GemmArgs a, unsigned mtiles, hipStream_t st) {
       return go(std::integral_constant<int, 512>{});
     }
   }
-  if constexpr (SWIGLU && (WL == kWlTiles || WL == kWlTilesF16)) {
-    if (a.few_rows && a.K == 2048)
+  if constexpr (WL == kWlPermute || (SWIGLU && (WL == kWlTiles || WL == kWlTilesF16))) {
+    if (a.few_rows && a.tile_rows <= 96 && a.K == 2048)
       return launch_rb<T, SWIGLU, GATHER, WL, 2048, 96, kRbNW, true>(a, mtiles, st);
   }
   if (a.tile_rows <= 96 && (a.K == 2048 || a.K == 512))
@@ -1159,7 +1164,8 @@ int routed_gemm(const RoutedGemm &r, hipStream_t st) {
   a.N = (int)r.n;
   a.K = (int)r.k;
   a.tile_rows = (int)r.bm;
-  a.few_rows = std::max(r.y_rows, r.form_rows) <= kFewRows * r.experts;
+  a.few_rows =
+      std::max(r.y_rows, r.form_rows) <= (r.q_tiles ? kFewRows : kFewRowsPlain) * r.experts;
   const unsigned mt = (unsigned)r.n_tiles;
   return r.dtype == LM_BF16 ? routed_dispatch<BF16>(a, mt, r.gather, r.swiglu, st)
                             : routed_dispatch<FP16>(a, mt, r.gather, r.swiglu, st);

@@ -611,6 +611,24 @@ def test_routed_moe_vs_oracle(dev, large):
                                              large), out)
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('tokens', [3, 20, 42])
+def test_routed_moe_forms_same_bits(dev, dtype, tokens):
+    """Few rows per expert (up to 21 on average: deep weight rings) give a token
+    the bits that it gets in a call of many (75), with tiles of 1 to 75 rows."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(16)
+    e, k = 16, 8
+    banks = [t for n, h in ((1024, 2048), (2048, 512)) for t in convert.quantize_g128(
+        torch.randn(e, n, h, generator=g, device=dev) * 0.02)]
+    x = torch.randn(150, 2048, generator=g, device=dev).to(dtype)
+    ids = torch.rand(150, e, generator=g, device=dev).topk(k, dim=1).indices
+    wts = torch.rand(150, k, generator=g, device=dev).to(dtype)
+    whole = gpu_routes.routed_moe(x, wts, ids, banks)
+    assert torch.equal(gpu_routes.routed_moe(x[:tokens], wts[:tokens], ids[:tokens], banks),
+                       whole[:tokens])
+
+
 def test_plan_routes_host_matches_device(dev):
     ids = _ids(seeded(16), 300, 256, 8, True)
     positions, segments = routing.plan_routes(ids, 256)
