@@ -58,7 +58,8 @@ __device__ __forceinline__ int id_rank(int id, int n, int lane) {
 }
 
 __global__ __launch_bounds__(256) void expert_table_kernel(ExpertsArgs a, int64_t *table) {
-  for (int j = threadIdx.x; j < a.n; j += 256) {
+  const int j = blockIdx.x * 256 + threadIdx.x;
+  if (j < a.n) {
     const int e = selected_id(a.ids, a.ids32, j, a.experts);
     int rank = 0;
     for (int i = 0; i < a.n; ++i) {
@@ -247,7 +248,7 @@ int experts_decode(const ExpertsArgs &a, hipStream_t st) {
 
 int check_selection(const void *ids, int ids_bytes, int64_t n, int64_t experts) {
   LM_REQUIRE(ids_bytes == 4 || ids_bytes == 8, LM_EINVAL, "expert ids must be int32 or int64");
-  LM_REQUIRE(n >= 0 && n < (1 << 20) && experts >= 1 && experts < (1LL << 31), LM_EINVAL,
+  LM_REQUIRE(n >= 0 && n < (1 << 20) && experts >= (n ? 1 : 0) && experts < (1LL << 31), LM_EINVAL,
              "invalid expert selection");
   LM_REQUIRE(n == 0 || ids, LM_EINVAL, "null pointer");
   return LM_OK;
@@ -279,7 +280,7 @@ extern "C" int lm_expert_table(const void *ids, int ids_bytes, int64_t n, int64_
   a.gu_ses = gu_s_expert_stride;
   a.dn_qes = dn_q_expert_stride;
   a.dn_ses = dn_s_expert_stride;
-  expert_table_kernel<<<1, 256, 0, as_stream(stream)>>>(a, table);
+  expert_table_kernel<<<cdiv(n, 256), 256, 0, as_stream(stream)>>>(a, table);
   return check_launch("expert_table_kernel");
 }
 

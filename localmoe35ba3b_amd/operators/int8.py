@@ -132,12 +132,13 @@ def build_descriptors(gate_up, down, ids):
 
     Returns an int64 [top_k, 5] table of (gate_up.q, gate_up.s, down.q,
     down.s) data pointers of each selected expert of the HBM bank plus its
-    slot, built by one kernel (no host read of the routing ids).  Ids in host
-    memory give the same table there; the operators take it only on the GPU.
+    slot, built on the device (no host read of the routing ids), by one kernel
+    for a token's.  Ids in host memory give the same table there; the operators
+    take it only on the GPU.
     """
-    if not ids.is_cuda:
+    if not ids.is_cuda or ids.numel() > _RANKED_IDS:
         experts, slots = torch.sort(ids.reshape(-1), stable=True)
-        experts = experts.to(torch.int64)
+        experts = experts.to(torch.int64).clamp(0, gate_up['q'].shape[0] - 1)
         columns = [t.data_ptr() + experts * (t.stride(0) * t.element_size())
                    for t in (gate_up['q'], gate_up['scale'], down['q'], down['scale'])]
         return torch.stack([*columns, slots], dim=1)
@@ -147,6 +148,11 @@ def build_descriptors(gate_up, down, ids):
     _lib.call('lm_expert_table', flat.data_ptr(), size, n, gate_up['q'].shape[0],
               *_bank_args(gate_up, down), table.data_ptr(), _lib.stream(flat.device))
     return table
+
+
+# The kernel compares every id with every other: 10 us for 64 ids, 52 for 512, 400
+# for 4096, where the sort and its arithmetic take about 90.
+_RANKED_IDS = 512
 
 
 @functools.lru_cache(maxsize=None)

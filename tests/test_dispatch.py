@@ -72,3 +72,11 @@ def test_router_digits_only_where_they_pay():
     for t, e, h in ((512, 256, 2048), (1024, 128, 2048), (16384, 17, 2048), (65536, 16, 4096),
                     (16384, 256, 256), (600, 256, 512), (2048, 256, 2016), (2048, 256, 8192)):
         assert not pays(t, e, h), (t, e, h)
+
+
+def test_descriptor_table_of_no_experts():
+    """An empty selection is a table without rows, also of an empty bank."""
+    lib = _lib.lib()
+    none = [None] * 4 + [0] * 4
+    assert lib.lm_expert_table(None, 8, 0, 0, *none, None, None) == _lib.LM_OK
+    assert lib.lm_expert_table(None, 8, 3, 0, *none, None, None) == _lib.LM_EINVAL

@@ -308,6 +308,16 @@ def test_experts_decode_forms(dev, n, hidden, inter, dtype, idt):
     assert torch.equal(out, ref)
 
 
+@pytest.mark.parametrize('n', [256, 257, 3000])
+def test_descriptor_table_of_many_ids(dev, n):
+    """More ids than one workgroup ranks, many of them equal."""
+    q, s = torch.zeros(50, 4, 128, dtype=torch.int8, device=dev), torch.zeros(50, 4, 1, device=dev)
+    bank = {'q': q, 'scale': s}
+    ids = torch.randint(0, 50, (n,), generator=seeded(n))
+    table = int8.build_descriptors(bank, bank, ids.to(dev))
+    assert torch.equal(table.cpu(), int8.build_descriptors(bank, bank, ids))
+
+
 # ------------------------------------------------------------- a6/a11/a12 glue
 def test_ordered_reduce_bit_exact(dev):
     gen = seeded(7)
