@@ -7,6 +7,27 @@ import pytest
 from localmoe35ba3b_amd import _lib
 
 GEMV, KSPLIT, STREAMED, LDS = range(4)
+KSPLIT_TILES = [(16, 16), (16, 32), (16, 64), (32, 32), (48, 32), (64, 32), (64, 64), (96, 32)]
+STREAMED_TILES = [(96, 128), (128, 128), (128, 256)]
+W8A8_TILES = [(32, 64), (64, 64), (64, 128), (128, 128)]
+# Sizes [m, n] that take every tile in both ways to deal them to the XCDs, ragged
+# in rows and columns; what the GPU tests run.
+DENSE = {
+    512: [(60, 17), (3, 17), (2100, 17), (3, 4104), (350, 600), (3, 8200), (3000, 34), (17, 4104),
+          (2100, 100), (33, 6000), (4000, 70), (60, 4104), (1200, 600), (60, 8200), (1700, 300),
+          (385, 1030), (1000, 1030), (97, 8200), (1300, 1030), (1030, 2050), (4000, 2040),
+          (1300, 6000)],
+    2048: [(60, 17), (3, 17), (2100, 17), (3, 4104), (350, 600), (3, 8200), (3000, 34), (17, 4104),
+           (1030, 200), (33, 6000), (4000, 70), (60, 4104), (1030, 600), (33, 8200), (2500, 200),
+           (65, 6000), (800, 3500), (200, 8200), (1700, 1030), (1030, 2050), (4000, 2040),
+           (1300, 6000)],
+    4096: [(60, 17), (3, 17), (2100, 17), (3, 4104), (350, 600), (3, 8200), (3000, 34), (17, 4104),
+           (1030, 200), (33, 6000), (4000, 70), (60, 4104), (800, 600), (33, 8200), (530, 900),
+           (65, 6000), (800, 3500), (200, 8200), (1700, 1030), (1030, 2050), (4000, 2040),
+           (1300, 6000)],
+}
+W8A8 = [(60, 34), (3, 34), (5000, 70), (33, 8200), (5000, 600), (260, 10000), (3000, 2050),
+        (600, 10000)]
 SIZES = [(m, n) for n in (16, 64, 128, 256, 512, 1000, 2048, 4096, 8192)
          for m in (9, 45, 130, 333, 700, 1023, 1024, 1100, 1900, 2048, 3000, 4096, 10000, 20000)]
 
@@ -21,6 +42,21 @@ def w8a8_form(m, n, k, swiglu=False):
     form = (ctypes.c_int64 * 4)()
     assert _lib.lib().lm_w8a8_gemm_form(m, n, k, int(swiglu), form) == _lib.LM_OK
     return tuple(form)
+
+
+@pytest.mark.parametrize('k', DENSE)
+def test_sizes_take_every_dense_tile(k):
+    forms = [linear_form(m, n, k) for m, n in DENSE[k]]
+    assert sorted(forms) == sorted(
+        (kernel, *tile, deal) for kernel, tiles in ((KSPLIT, KSPLIT_TILES),
+                                                    (STREAMED, STREAMED_TILES))
+        for tile in tiles for deal in (0, 1))
+
+
+@pytest.mark.parametrize('swiglu', [False, True])
+def test_sizes_take_every_w8a8_tile(swiglu):
+    forms = [w8a8_form(m, n, 128, swiglu) for m, n in W8A8]
+    assert sorted(forms) == sorted((LDS, *tile, deal) for tile in W8A8_TILES for deal in (0, 1))
 
 
 def _rounds(m, n, rows, cols):

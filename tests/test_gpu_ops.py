@@ -15,9 +15,12 @@ from localmoe35ba3b_amd.operators import int8, routing, w8a8
 from localmoe35ba3b_amd.runtime import gpu_routes, prefill
 from localmoe35ba3b_amd.runtime.stack import zipf_bias
 from oracle import moe_oracle as O
+from tests import test_dispatch
 from tests.conftest import BF16_TOL, assert_close, seeded
 
 pytestmark = pytest.mark.gpu
+
+LM_HEAD_N = 248320  # vocabulary of the 35B-A3B configuration
 
 
 def bf16_rand(shape, gen, scale=1.0):
@@ -122,10 +125,10 @@ def test_w8a8_gemm_bit_exact(dev, m, n, rows):
                                    (33, 130, 384), (700, 4096, 128), (1000, 1100, 256),
                                    (1025, 4100, 128), (2100, 4000, 128)])
 def test_w8a8_gemm_tiles_bit_exact(dev, m, n, k, dtype):
-    """Every tile of the W8A8 GEMM (32 x 64 to 128 x 128, chosen by size) and
-    the K-parallel form of up to 16 rows, with ragged rows and columns: the
-    outputs of a sample of rows equal the oracle's bit for bit, SwiGLU within
-    the rounding of its exponential."""
+    """The W8A8 GEMM's tiles of 32 x 64 to 64 x 128 and the K-parallel form of up to
+    16 rows, with ragged rows and columns: the outputs of a sample of rows equal
+    the oracle's bit for bit, SwiGLU the operator's on them (every tile:
+    test_w8a8_gemm_every_tile)."""
     rnd = O.bf16 if dtype == torch.bfloat16 else O.fp16
     gen = seeded(m + n)
     x = torch.randn(m, k, generator=gen).to(dtype)
@@ -181,12 +184,12 @@ def test_w8a8_grouped_decode_bit_exact(dev):
                                    (1057, 4096, 2048), (1100, 1000, 512), (3000, 3000, 2048),
                                    (4096, 2048, 512)])
 def test_w8a16_linear(dev, m, n, k):
-    """Every GEMM path of int8.linear against the oracle: the GEMV (m <= 8),
-    96-row tiles, 128-row tiles from m = 1024 (1057 and 1100 end in partial
-    tiles of 33 and 76 rows), the wide 8-wave 256-column tiles where they give
-    every CU a tile (2048 x 4096, 3000 x 3000 with a partial row tile of 56
-    rows and a partial column tile of 184 columns, and K = 512), the generic
-    kernel at K = 384."""
+    """int8.linear against the oracle on real-valued inputs: the GEMV, K-split
+    tiles, 128-row tiles (1057 ends in a partial tile of 33 rows), the wide
+    8-wave 256-column tiles where they give every CU a tile (2048 x 4096, 3000 x
+    3000 with a partial row tile of 56 rows and a partial column tile of 184
+    columns, and K = 512), the generic kernel at K = 384 (every tile:
+    test_w8a16_linear_every_tile)."""
     gen = seeded(m + n)
     x = bf16_rand((m, k), gen)
     wq, ws = O.quantize_weight((torch.randn(n, k, generator=gen) * 0.02).numpy())
@@ -218,10 +221,10 @@ def test_w8a16_linear_exact(dev, m, n):
     (3, 1000, 4096), (17, 600, 4096), (65, 2050, 4096), (260, 2040, 4096), (1100, 300, 4096),
     (1057, 4096, 4096), (2000, 4100, 4096)])
 def test_w8a16_linear_ksplit_exact(dev, m, n, k, dtype):
-    """Every K-split tile shape at each K it serves (16 to 96 rows by 16 to 64
-    columns, ragged in both), and the tall tiles at K = 4096: integers and
-    powers of two make every sum exact in fp32 (below 2^24 units of 2^-6), so
-    the result is the rounded exact product whatever the order of the sum."""
+    """K-split tiles at each K they serve, ragged in rows and columns, and the tall
+    tiles at K = 4096: integers and powers of two make every sum exact in fp32
+    (below 2^24 units of 2^-6), so the result is the rounded exact product
+    whatever the order of the sum."""
     g = np.random.default_rng(m + n + k)
     x = g.integers(-8, 9, size=(m, k)).astype(np.float32)
     q = g.integers(-127, 128, size=(n, k)).astype(np.int8)
@@ -232,6 +235,58 @@ def test_w8a16_linear_ksplit_exact(dev, m, n, k, dtype):
     w = q.astype(np.float32).reshape(n, -1, 128) * s[..., None]
     exact = torch.from_numpy(x) @ torch.from_numpy(w.reshape(n, k)).t()
     assert torch.equal(y.cpu(), exact.to(dtype))
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('m,n,k', [(m, n, k) for k, sizes in test_dispatch.DENSE.items()
+                                   for m, n in sizes])
+def test_w8a16_linear_every_tile(dev, m, n, k, dtype):
+    """Every K-split and register-streamed tile at each K, dealt to the XCDs both
+    ways, ragged in rows and columns (test_dispatch.py checks that these sizes take
+    them): every sum is exact in fp32, as above."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(m + n + k)
+    x = torch.randint(-8, 9, (m, k), generator=g, device=dev)
+    q = torch.randint(-127, 128, (n, k), generator=g, device=dev, dtype=torch.int8)
+    s = torch.full((n, k // 128), 2.0 ** -6, device=dev)
+    s[::3, ::2] = 2.0 ** -5
+    y = int8.linear(x.to(dtype), q, s)
+    w = (q.double().view(n, -1, 128) * s.double()[..., None]).view(n, k)
+    assert torch.equal(y, (x.double() @ w.t()).to(dtype))
+
+
+def test_lm_head_few_rows_exact(dev):
+    """Four rows by the vocabulary run K-split tiles over 3880 column tiles."""
+    assert test_dispatch.linear_form(4, LM_HEAD_N, 2048) == (test_dispatch.KSPLIT, 16, 64, 1)
+    g = torch.Generator(device=dev)
+    g.manual_seed(4)
+    x = torch.randint(-8, 9, (4, 2048), generator=g, device=dev)
+    q = torch.randint(-127, 128, (LM_HEAD_N, 2048), generator=g, device=dev, dtype=torch.int8)
+    s = torch.full((LM_HEAD_N, 16), 2.0 ** -6, device=dev)
+    y = int8.linear(x.to(torch.bfloat16), q, s)
+    for r in range(0, LM_HEAD_N, 1 << 16):
+        exact = x.double() @ (q[r:r + (1 << 16)].double() * 2.0 ** -6).t()
+        assert torch.equal(y[:, r:r + (1 << 16)], exact.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('swiglu', [False, True])
+@pytest.mark.parametrize('m,n', test_dispatch.W8A8)
+def test_w8a8_gemm_every_tile(dev, m, n, swiglu, dtype):
+    """Every tile of the W8A8 GEMM, dealt to the XCDs both ways, ragged in rows and
+    columns, with one and three K groups: a sample of rows equals the oracle's bit for
+    bit, with SwiGLU the operator's on them."""
+    rnd = O.bf16 if dtype == torch.bfloat16 else O.fp16
+    for k in (128, 384):
+        gen = seeded(m + n + k)
+        x = torch.randn(m, k, generator=gen).to(dtype)
+        wq, ws = O.quantize_weight((torch.randn(n, k, generator=gen) * 0.02).numpy())
+        xq, xs = w8a8.quantize(x.to(dev))
+        y = w8a8.gemm(xq, xs, torch.from_numpy(wq).to(dev), torch.from_numpy(ws).to(dev), swiglu,
+                      out_dtype=dtype)
+        sel = np.unique(np.r_[0, m - 1, np.random.default_rng(m).integers(0, m, 8)])
+        ref = torch.from_numpy(O.w8a8_linear(x.float().numpy()[sel], wq, ws, rnd)).to(dtype).to(dev)
+        assert torch.equal(y[torch.from_numpy(sel).to(dev)], int8.swiglu(ref) if swiglu else ref)
 
 
 @pytest.mark.parametrize('m', [64, 1030])
@@ -709,9 +764,6 @@ def test_routed_reduce_batches(dev, k, n):
     for tok in range(t):
         ref = O.ordered_combine(npf(v)[ro[tok]], w.numpy()[tok, rs[tok]], O.fp16)
         assert np.array_equal(npf(y[tok]), ref)
-
-
-LM_HEAD_N = 248320  # vocabulary of the 35B-A3B configuration
 
 
 @pytest.mark.parametrize('m', [1, 2])
