@@ -89,8 +89,9 @@ int lm_act_quant_g128(const void *x, int x_dtype, int8_t *q, float *s,
  * fp32 accumulation, y in the activation dtype.  The size selects
  * the kernel: the HBM streaming GEMV (one or two rows, and up to 8 where the
  * K-split tiles do not serve), K-split MFMA tiles, or the register-streamed
- * MFMA tiles of many rows.  large_tile only selects a tile height, where K
- * has no tile of its own.  Replaces int8.linear / int8._linear (int8.py:9-37). */
+ * MFMA tiles of many rows (K = 512, 2048, 4096; tiles that dequantize into LDS for
+ * other K).  large_tile is the reference's flag; it has no effect, the size
+ * chooses.  Replaces int8.linear / int8._linear (int8.py:9-37). */
 int lm_w8a16_linear(const void *x, const int8_t *q, const float *s, void *y,
                     int64_t m, int64_t n, int64_t k, int dtype, int large_tile,
                     void *stream);

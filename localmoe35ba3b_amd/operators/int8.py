@@ -31,7 +31,7 @@ def linear(x, q, scale, large_tile=False):
 
     x: CUDA bf16/fp16 [..., K]; q int8 [N, K]; scale fp32 [N, K/128].
     One or two rows run the HBM-streaming GEMV, more the MFMA tiles their size
-    selects; large_tile selects the taller tile like the reference flag.
+    selects; large_tile is taken like the reference's flag and has no effect.
     """
     if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError('W8A16 requires CUDA FP16/BF16 activations')
@@ -197,10 +197,10 @@ class Int8Experts(torch.nn.Module):
             banks = [self.gate_up['q'], self.gate_up['scale'], self.down['q'], self.down['scale']]
             return gpu_routes.routed_moe(x, top_k_weights, top_k_index.contiguous(), banks,
                                          self.large_tile)
-        hidden, intermediate = x.shape[-1], self.down['q'].shape[-1]
+        hidden, intermediate, n = x.shape[-1], self.down['q'].shape[-1], top_k_index.numel()
         if ((build_descriptors, grouped_linear, swiglu, ordered_reduce) == _w8a16_decode
-                and _decode_fits(top_k_index.numel(), hidden, intermediate)):
-            return self._decode(x, top_k_index, top_k_weights, hidden, intermediate)
+                and _decode_fits(n, hidden, intermediate)):
+            return self._decode(x, top_k_index, n, top_k_weights, hidden, intermediate)
         table = build_descriptors(self.gate_up, self.down, top_k_index)
         experts = table.shape[0]
         gu = grouped_linear(x, table, experts, 2 * intermediate, 0, True)
@@ -208,13 +208,12 @@ class Int8Experts(torch.nn.Module):
         values = grouped_linear(h, table, experts, hidden, 2, False)
         return ordered_reduce(values, table, top_k_weights)
 
-    def _decode(self, x, ids, weights, hidden, intermediate):
+    def _decode(self, x, ids, n, weights, hidden, intermediate):
         """One token, W8A16: gate_up + SwiGLU, then down + combine, two launches
         with the results of the separate operators."""
         if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16):
             raise ValueError('W8A16 requires CUDA FP16/BF16 activations')
         flat, size = _selection(ids)
-        n = flat.numel()
         x, weights = x.contiguous(), _check_weights(weights, n)
         h = x.new_empty((n, intermediate))
         out = x.new_empty((1, hidden))
