@@ -1050,17 +1050,15 @@ struct DenseForm {
 };
 
 static DenseForm dense_form(int64_t m, int64_t n, int64_t k) {
+  // One or two rows stream the weights through the GEMV (lm_head
+  // [248320, 2048]: 77 against 92 us on K-split tiles); from three rows on
+  // the GEMV's dot products cost more than the weights (200 against 93 us;
+  // at N = 4096 and 8 rows 6.9 against 4.1 us), and at K = 512 one round of
+  // K-split tiles is the shorter chain (2.6 against 3.4 us).
+  if (m <= 2 && !(k == 512 && n <= 256 * 16)) return DenseForm{LM_LINEAR_GEMV};
   const KsPlan ks = ksplit_plan(m, n, k);
-  DenseForm f{LM_LINEAR_KSPLIT, ks, ks.rows, ks.cols, ks.by_columns};
-  if (m <= 8) {
-    // One or two rows stream the weights through the GEMV (lm_head
-    // [248320, 2048]: 77 against 92 us on K-split tiles); from three rows on
-    // the GEMV's dot products cost more than the weights (200 against 93 us;
-    // at N = 4096 and 8 rows 6.9 against 4.1 us), and at K = 512 one round of
-    // K-split tiles is the shorter chain (2.6 against 3.4 us).
-    if (ks.shape >= 0 && (m > 2 || (k == 512 && n <= 256 * 16))) return f;
-    return DenseForm{LM_LINEAR_GEMV, ks, 0, 0, false};
-  }
+  const DenseForm f{LM_LINEAR_KSPLIT, ks, ks.rows, ks.cols, ks.by_columns};
+  if (m <= 8) return ks.shape >= 0 ? f : DenseForm{LM_LINEAR_GEMV};
   // Other K: the LDS-dequant kernel.
   if (ks.shape < 0) return DenseForm{LM_LINEAR_LDS, ks, 128, kBN, false};
   // K = 512, 2048 or 4096: small tiles whose waves split K (ksplit.hip) or the

@@ -231,8 +231,10 @@ KsPlan ksplit_plan(int64_t m, int64_t n, int64_t k) {
   for (int i = 0; i < kKsCount; ++i) {
     const int ms = kKsShapes[i][0], ni = kKsShapes[i][1];
     const int64_t mt = cdiv(m, 16 * ms), nt = cdiv(n, 16 * ni);
-    const XcdDeal deal = xcd_deal(m, n, mt, nt, 16 * ms, false, in_l2 ? 0 : 2);
     const double round = 0.18 * ms * ni + 0.8 * (ms + ni) * (double)k / 2048.0;
+    // a small call's host side: no deal is better than one tile on every CU in turn
+    if (best.shape >= 0 && 1.8 + (double)((mt * nt + 255) / 256) * round >= best.cost) continue;
+    const XcdDeal deal = xcd_deal(m, n, mt, nt, 16 * ms, false, in_l2 ? 0 : 2);
     const double cost = 1.8 + deal.rounds * round * (deal.by_columns && !in_l2 ? 1.1 : 1.0);
     if (best.shape < 0 || cost < best.cost)
       best = KsPlan{i, cost, 16 * ms, 16 * ni, deal.by_columns};
