@@ -233,8 +233,8 @@ struct W8A8Form {
 // The tile with the smallest estimated time at K = 2048 (all scale with K
 // alike): a + b r us for r rounds of a tile per CU, measured from r = 1 to 16
 // ([64, 2048] by [4096, 2048]: 8.7 us in 32 x 64 tiles, 25 in 128 x 128; [700,
-// 2048] by [4096, 2048]: 19.5 us in 64 x 64, 26 in 128 x 128; [2048, 2048] by
-// [4096, 2048]: 36 us in 128 x 128, 42 in 64 x 64).  In SwiGLU mode a tile's
+// 2048] by [4096, 2048]: 17.7 us in 64 x 64, 24.5 in 128 x 128; [2048, 2048] by
+// [4096, 2048]: 35 us in 128 x 128, 42 in 64 x 64).  In SwiGLU mode a tile's
 // columns are pairs of weight rows.
 W8A8Form w8a8_form(int64_t m, int64_t n, bool swiglu) {
   constexpr int tiles[4][2] = {{32, 64}, {64, 64}, {64, 128}, {128, 128}};

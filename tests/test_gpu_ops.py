@@ -486,10 +486,11 @@ def _direct_router(x, w, k, bias):
     (600, 256, 2048, 'outliers'), (520, 256, 1024, 'wide'), (515, 100, 4096, 'edges'),
     (550, 256, 2048, 'ties')])
 def test_router_digits(dev, t, e, h, kind):
-    """The int8-digit form (more than 512 tokens) against the fp64 form, bit for
-    bit: ragged tiles, one to many K blocks, rows whose values leave the
+    """router_topk of more than 512 tokens, which takes the int8-digit form where
+    that pays (test_router_digit_residues runs it at every size), against the fp64
+    form, bit for bit: ragged tiles, one to many K blocks, rows whose values leave the
     23-bit grid ('outliers': a few channels 300 times the others; 'wide': values
-    from 2^-40 to 2^20, every logit open), rows of zeros, subnormals,
+    from 2^-40 to 2^20, every logit open by the grid alone), rows of zeros, subnormals,
     infinities and NaN ('edges'), and exact ties at bf16 rounding boundaries."""
     assert _lib.lib().lm_router_workspace_bytes(t, e, h) > 0
     g = torch.Generator(device=dev)
