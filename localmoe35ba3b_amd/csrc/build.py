@@ -38,7 +38,7 @@ COMMON = ['-O3', '-std=c++17', '-fPIC', f'--offload-arch={ARCH}', '-ffp-contract
 # took 55.4 us instead of 50.7.
 EXTRA = {'w8a8_gemm.hip': ['-falign-loops=64'],
          'moe.hip': ['-mllvm', '-amdgpu-kernarg-preload-count=6',
-                      '-mllvm', '-amdgpu-mfma-vgpr-form=1']}
+                     '-mllvm', '-amdgpu-mfma-vgpr-form=1']}
 
 
 def hipcc():
